@@ -68,7 +68,10 @@ enum rebop_kernel_kind {
   REBOP_KERNEL_PERSISTENT = 2, /* lanes refill from an atomic trajectory queue */
   REBOP_KERNEL_LDS = 3,        /* counts in LDS: 256 bytes per species (int32; 512 with
                                   REBOP_KERNEL_WIDE, 128 with int16 counts) and 16 per
-                                  reaction must fit one workgroup's LDS (160 KB) */
+                                  reaction must fit one workgroup's LDS (160 KB).  Also
+                                  reported where AUTO or a job batch ran the incremental
+                                  kernel (eight lanes per trajectory, counts in LDS), whose
+                                  results are the same */
   /* flag: the network compiled into the kernel (run-time compilation,
    * cached); combine with PLAIN or PERSISTENT */
   REBOP_KERNEL_SPECIALIZED = 16,
@@ -103,7 +106,9 @@ enum rebop_kernel_kind {
    * smaller LDS lets more waves share a CU (large networks: otherwise the
    * registers bound the waves, and int32 runs as fast without the risk of a
    * rerun); a launch that meets a larger count stops early and is rerun
-   * with int32 counts (then int64).  REBOP_LDS_COMPACT=0 in the environment
+   * with int32 counts (then int64).  The incremental kernel always keeps
+   * int32 and reports this flag where those counts stayed in the int16
+   * range.  REBOP_LDS_COMPACT=0 in the environment
    * never starts at int16, =1 does whenever the initial counts fit. */
   REBOP_KERNEL_COMPACT = 512
 };

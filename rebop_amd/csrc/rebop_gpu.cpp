@@ -47,6 +47,14 @@ hipError_t launch_lds(const rebop_dev_job *jobs, const rebop_dev_item *items, ui
                       uint32_t rec_word_off, int width, bool expr, bool grec, bool rerun,
                       hipStream_t stream);
 
+size_t inc_lds_bytes(uint32_t smax, uint32_t nblk_max, uint32_t rmax, uint32_t depth, bool store);
+hipError_t inc_occupancy(size_t lds, bool expr, bool store, int *blocks_per_cu);
+hipError_t launch_inc(const rebop_dev_job *jobs, const uint32_t *tickets, uint32_t n_tickets,
+                      unsigned long long *counters, unsigned long long *job_events,
+                      unsigned long long *job_queue, int blocks, uint32_t smax, uint32_t nblk_max,
+                      uint32_t rmax, uint32_t depth, bool expr, bool store, bool rerun,
+                      hipStream_t stream);
+
 } // namespace rebop
 
 namespace {
@@ -177,6 +185,10 @@ constexpr int kRetryWide = -1;
 // counts' exact range (rerun it on the LDS kernel's int64 counts)
 constexpr int kRetryExact = -2;
 
+// launch_run's `kernel`: the LDS kernel or the incremental one (AUTO's choice
+// between the two), not REBOP_KERNEL_LDS itself
+constexpr int kKernelAnyLds = 1 << 20;
+
 // Draws per trajectory after which a run whose horizon is not finite (tmax
 // = +inf or NaN) stops a trajectory that never reaches an absorbing state,
 // when the handle sets no cap of its own.
@@ -207,6 +219,11 @@ struct rebop_gillespie {
   double tune_occ = 1.0;
   // the network part of an LDS-kernel job (sparse jump, checkpoint blocks)
   rebop_dev_job job{};
+  // the incremental kernel: whether some jump moves a count by more than its
+  // update list can say (it then stores the propensities), and its deepest
+  // expression stack
+  bool inc_store = false;
+  uint32_t inc_depth = 0;
   DevBuf djobs, ditems;
   // network-specialised kernels (run-time compiled), rebuilt when reactions
   // change: [0] plain, [1] with the draw-cap checks (compiled when first needed)
@@ -244,6 +261,123 @@ int check_x0(const int64_t *x, size_t n) {
                                        " is beyond the exactly simulated range |n| <= 2^52");
   }
   return REBOP_OK;
+}
+
+// The incremental kernel's tables (layout in ssa_layout.h), and whether it
+// runs this network at all: mass-action reactions of at most two factors with
+// non-negative constants whose jumps cannot take a count below zero, rate
+// expressions (their values are checked as they come), jumps that fit a
+// record, at most 4096 reactions.  Anything else runs on the other kernels.
+struct IncTables {
+  bool ok = false, store = false;
+  uint32_t bsh = 3, depth = 0;
+  std::vector<uint32_t> rec, dep, tok;
+};
+
+constexpr size_t kIncMaxReactions = 4096; // 64 blocks of at most 64
+constexpr size_t kIncMaxDep = 1u << 22;
+
+// One expression's tokens.  An operand pushed just before a binary operation
+// is read by the operation itself, so the push goes away; the operations and
+// their order stay.  Returns the deepest stack.
+uint32_t inc_expression(const Reaction &x, std::vector<uint32_t> *tok) {
+  uint32_t depth = 0, deepest = 0;
+  for (size_t i = 0; i < x.expr.size(); ++i) {
+    uint32_t op = REBOP_EXPR_OPCODE(x.expr[i]), src = REBOP_TOK_STACK, row = 0;
+    double c = 0.0;
+    if (op == REBOP_OP_CONST || op == REBOP_OP_SPECIES) {
+      const uint32_t arg = REBOP_EXPR_ARG(x.expr[i]);
+      src = op == REBOP_OP_CONST ? REBOP_TOK_CONST : REBOP_TOK_SPECIES;
+      if (op == REBOP_OP_CONST) c = x.consts[arg];
+      else row = arg + 1u;
+      const uint32_t next = i + 1 < x.expr.size() ? REBOP_EXPR_OPCODE(x.expr[i + 1]) : 0u;
+      if (next >= REBOP_OP_ADD && next <= REBOP_OP_MIN) {
+        op = next;
+        ++i;
+      } else {
+        op = REBOP_OP_CONST; // push
+        depth += 1;
+        deepest = std::max(deepest, depth);
+      }
+    } else if (op >= REBOP_OP_ADD && op <= REBOP_OP_MIN) {
+      depth -= 1;
+    }
+    uint64_t b;
+    std::memcpy(&b, &c, sizeof b);
+    tok->insert(tok->end(), {op | (src << 8), row, (uint32_t)b, (uint32_t)(b >> 32)});
+  }
+  return deepest;
+}
+
+// `rec`: the reaction records; an expression's gets its token range.
+IncTables inc_tables(const rebop_gillespie *g, std::vector<uint32_t> &rec,
+                     const std::vector<uint32_t> &jrec) {
+  IncTables t;
+  const uint32_t S = g->S, R = (uint32_t)g->rx.size();
+  if (g->system || R == 0 || R > kIncMaxReactions) return t;
+  std::vector<std::vector<uint32_t>> readers(S); // reactions whose propensity reads a species
+  for (uint32_t r = 0; r < R; ++r) {
+    const Reaction &x = g->rx[r];
+    const uint32_t w3 = rec[(size_t)REBOP_REC_WORDS * r + 3];
+    if ((w3 & REBOP_REC_SLOW_JUMP) || !(x.k >= 0.0)) return t;
+    auto reads = [&](uint32_t s) {
+      if (readers[s].empty() || readers[s].back() != r) readers[s].push_back(r);
+    };
+    if (!x.expr.empty()) {
+      for (uint32_t tk : x.expr)
+        if (REBOP_EXPR_OPCODE(tk) == REBOP_OP_SPECIES) reads(REBOP_EXPR_ARG(tk));
+      continue;
+    }
+    if (w3 & REBOP_REC_SLOW_FACTORS) return t;
+    for (auto &e : x.entries) reads(e.first);
+    for (uint32_t s = 0; s < S; ++s) {
+      if (x.diff[s] >= 0) continue;
+      uint32_t seen = 0, order = 0;
+      for (auto &e : x.entries)
+        if (e.first == s) {
+          seen++;
+          order = e.second;
+        }
+      if (seen != 1 || (int64_t)order < -x.diff[s]) return t;
+    }
+  }
+  while (((R - 1u) >> t.bsh) >= 64u) t.bsh += 1u;
+  t.rec.assign((size_t)REBOP_IREC_WORDS * R, 0u);
+  std::vector<uint32_t> mark(R, ~0u);
+  for (uint32_t k = 0; k < R; ++k) {
+    const Reaction &x = g->rx[k];
+    uint32_t *w = t.rec.data() + (size_t)REBOP_IREC_WORDS * k;
+    std::memcpy(w, jrec.data() + (size_t)REBOP_JREC_WORDS * k, sizeof(uint32_t) * REBOP_JREC_WORDS);
+    w[4] = (uint32_t)t.dep.size();
+    for (uint32_t s = 0; s < S; ++s) {
+      if (x.diff[s] == 0) continue;
+      for (uint32_t r : readers[s]) {
+        if (mark[r] == k) continue;
+        mark[r] = k;
+        uint32_t e = r;
+        for (uint32_t q = 0; q < 2; ++q) {
+          const uint32_t row = rec[(size_t)REBOP_REC_WORDS * r + 2 + q] >> 16;
+          const int64_t d = row && g->rx[r].expr.empty() ? x.diff[row - 1u] : 0;
+          if (d < -128 || d > 127) t.store = true;
+          e |= ((uint32_t)d & 0xffu) << (16 + 8 * q);
+        }
+        t.dep.push_back(e);
+      }
+    }
+    w[5] = (uint32_t)t.dep.size() - w[4];
+    if (t.dep.size() > kIncMaxDep) return t;
+  }
+  for (uint32_t r = 0; r < R; ++r) {
+    if (g->rx[r].expr.empty()) continue;
+    uint32_t *w = rec.data() + (size_t)REBOP_REC_WORDS * r;
+    w[0] = (uint32_t)(t.tok.size() / 4u);
+    t.depth = std::max(t.depth, inc_expression(g->rx[r], &t.tok));
+    w[1] = (uint32_t)(t.tok.size() / 4u);
+    t.store = true;
+  }
+  if (!t.tok.empty()) t.tok.insert(t.tok.end(), 4u, 0u); // read ahead of the last token
+  t.ok = true;
+  return t;
 }
 
 // Packs the network into one device buffer (layout in ssa_layout.h).
@@ -369,6 +503,7 @@ int upload_net(rebop_gillespie *g) {
       }
     }
   }
+  IncTables inc = inc_tables(g, rec, jrec);
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t ok = 0;
   const size_t ofb = ok + al(sizeof(double) * R);
@@ -388,7 +523,10 @@ int upload_net(rebop_gillespie *g) {
   const size_t otb = oek + al(sizeof(double) * EK);
   const size_t ots = otb + al(sizeof(uint32_t) * (R + 1));
   const size_t otm = ots + al(sizeof(uint32_t) * TS);
-  const size_t total = otm + al(sizeof(uint32_t) * TS);
+  const size_t oir = otm + al(sizeof(uint32_t) * TS);
+  const size_t oid = oir + al(sizeof(uint32_t) * inc.rec.size());
+  const size_t oit = oid + al(sizeof(uint32_t) * inc.dep.size());
+  const size_t total = oit + al(sizeof(uint32_t) * inc.tok.size());
   std::vector<unsigned char> host(total, 0);
   std::memcpy(host.data() + ojb, jb.data(), sizeof(uint32_t) * (R + 1));
   if (J) std::memcpy(host.data() + ojs, js.data(), sizeof(uint32_t) * J);
@@ -411,6 +549,13 @@ int upload_net(rebop_gillespie *g) {
       std::memcpy(host.data() + ots, tsp.data(), sizeof(uint32_t) * TS);
       std::memcpy(host.data() + otm, tmul.data(), sizeof(uint32_t) * TS);
     }
+  }
+  if (inc.ok) {
+    std::memcpy(host.data() + oir, inc.rec.data(), sizeof(uint32_t) * inc.rec.size());
+    if (!inc.dep.empty())
+      std::memcpy(host.data() + oid, inc.dep.data(), sizeof(uint32_t) * inc.dep.size());
+    if (!inc.tok.empty())
+      std::memcpy(host.data() + oit, inc.tok.data(), sizeof(uint32_t) * inc.tok.size());
   }
   HIP_TRY(g->dnet.ensure(total));
   HIP_TRY(hipMemcpy(g->dnet.p, host.data(), total, hipMemcpyHostToDevice));
@@ -456,6 +601,14 @@ int upload_net(rebop_gillespie *g) {
     jt.sys_species = (const uint32_t *)(base + ots);
     jt.sys_mult = (const uint32_t *)(base + otm);
   }
+  if (inc.ok) {
+    jt.inc_bsh = inc.bsh;
+    jt.inc_rec = (const uint32_t *)(base + oir);
+    jt.inc_dep = (const uint32_t *)(base + oid);
+    if (!inc.tok.empty()) jt.inc_tok = (const uint32_t *)(base + oit);
+  }
+  g->inc_store = inc.store;
+  g->inc_depth = inc.depth;
   g->job = jt;
   g->dirty = false;
   g->dev_id = cur;
@@ -809,6 +962,101 @@ int enqueue_lds(const std::vector<rebop_dev_job> &jobs, const std::vector<double
   return REBOP_OK;
 }
 
+// The incremental kernel's launch for a set of jobs.
+struct IncShape {
+  bool ok = false, expr = false, store = false;
+  uint32_t smax = 1, rmax = 1, nblk = 1, depth = 0;
+  int per_cu = 0; // waves per CU
+};
+
+// Whether the incremental kernel is the faster one for mass-action jobs.  Its
+// cost of an event hardly depends on the number of reactions, the LDS
+// kernel's grows with it; but the LDS kernel runs 64 trajectories a wave, so
+// a launch that fills its lanes (131072 resident trajectories) pays less per
+// event for a small network.  Measured, events/s incremental : LDS kernel --
+// 16384 trajectories, 40 species: 20 reactions 2.9e9 : 2.6e9; 65536: 40
+// reactions 4.0e9 : 5.0e9, 65 reactions 4.7e9 : 4.7e9, 96 reactions 4.9e9 :
+// 4.1e9; 262144: 96 reactions 6.0e9 : 6.6e9, 130 reactions 6.9e9 : 6.2e9.
+// The line through those ties is R = n / 1024, up to 128 reactions where the
+// lanes are full; a batch counts its mean reactions per trajectory.
+bool inc_pays(const std::vector<rebop_dev_job> &jobs) {
+  double n = 0.0, nr = 0.0;
+  for (auto &j : jobs) {
+    n += (double)j.n_traj;
+    nr += (double)j.n_traj * (double)j.R;
+  }
+  return nr >= n * std::min(128.0, n / 1024.0);
+}
+
+// Whether the incremental kernel runs these jobs, and how.
+IncShape inc_shape(const std::vector<rebop_dev_job> &jobs, bool store, uint32_t depth) {
+  IncShape s;
+  s.store = store;
+  s.depth = depth;
+  for (auto &j : jobs) {
+    if (!j.inc_rec || j.mode != REBOP_MODE_GRID || j.st_x || j.draw_cap) return s;
+    s.smax = std::max(s.smax, j.S);
+    s.rmax = std::max(s.rmax, j.R);
+    s.nblk = std::max(s.nblk, ((j.R - 1u) >> j.inc_bsh) + 1u);
+    s.expr = s.expr || j.inc_tok;
+  }
+  auto waves = [&](bool st) {
+    const size_t lds = rebop::inc_lds_bytes(s.smax, s.nblk, s.rmax, s.depth, st);
+    int n = 0;
+    if (lds > g_dev.lds_max || rebop::inc_occupancy(lds, s.expr, st, &n) != hipSuccess) return 0;
+    return n;
+  };
+  s.per_cu = waves(s.store);
+  if (!s.store) {
+    // stored propensities save the evaluation of the old ones; they are kept
+    // where their LDS costs no waves
+    const int st = waves(true);
+    if (st >= s.per_cu) {
+      s.per_cu = st;
+      s.store = true;
+    }
+  }
+  s.ok = s.per_cu > 0 && (s.expr || inc_pays(jobs));
+  return s;
+}
+
+// Uploads the job and ticket tables and enqueues the incremental kernel.
+int enqueue_inc(const std::vector<rebop_dev_job> &jobs, const std::vector<double> &cost,
+                const IncShape &shape, DevBuf *djobs, DevBuf *dtickets, unsigned long long *counters,
+                unsigned long long *job_events, unsigned long long *job_queue, bool rerun,
+                hipStream_t stream) {
+  const uint64_t resident = (uint64_t)shape.per_cu * (uint64_t)g_dev.cus;
+  // a job's tickets: eight trajectories each, never more than run at once (a
+  // wave takes its job's trajectories until none is left)
+  auto count = [&](const rebop_dev_job &j) { return std::min((j.n_traj + 7u) / 8u, resident); };
+  std::vector<uint32_t> tickets;
+  uint64_t n = 0;
+  if (jobs.size() == 1) {
+    n = count(jobs[0]);
+  } else {
+    std::vector<uint32_t> order(jobs.size());
+    for (uint32_t j = 0; j < order.size(); ++j) order[j] = j;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](uint32_t a, uint32_t b) { return cost[a] > cost[b]; });
+    for (uint32_t j : order) tickets.insert(tickets.end(), count(jobs[j]), j);
+    n = tickets.size();
+  }
+  if (n == 0) return REBOP_OK;
+  if (n > 0xffffffffull) return fail(REBOP_ERR_VALUE, "too many work items");
+  const size_t jbytes = sizeof(rebop_dev_job) * jobs.size();
+  HIP_TRY(djobs->ensure(jbytes));
+  HIP_TRY(hipMemcpyAsync(djobs->p, jobs.data(), jbytes, hipMemcpyHostToDevice, stream));
+  if (!tickets.empty()) {
+    HIP_TRY(dtickets->ensure(sizeof(uint32_t) * n));
+    HIP_TRY(hipMemcpyAsync(dtickets->p, tickets.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, stream));
+  }
+  HIP_TRY(rebop::launch_inc((const rebop_dev_job *)djobs->p,
+                            tickets.empty() ? nullptr : (const uint32_t *)dtickets->p, (uint32_t)n,
+                            counters, job_events, job_queue, (int)std::min(n, resident), shape.smax,
+                            shape.nblk, shape.rmax, shape.depth, shape.expr, shape.store, rerun, stream));
+  return REBOP_OK;
+}
+
 // Reads the counters of a finished launch into `stats` (waits for the stream).
 int finish_stats(rebop_stats *stats, unsigned long long *counters, const EventPair &ev, int kind,
                  hipStream_t stream, uint64_t draw_cap) {
@@ -820,6 +1068,8 @@ int finish_stats(rebop_stats *stats, unsigned long long *counters, const EventPa
   stats->events = ctr[REBOP_CTR_EVENTS];
   stats->draws = ctr[REBOP_CTR_DRAWS];
   stats->trajectories = ctr[REBOP_CTR_TRAJ];
+  // the incremental kernel keeps int32: what it reports is the width its counts needed
+  if (ctr[REBOP_CTR_FLAGS] & REBOP_FLAG_PAST16) kind &= ~REBOP_KERNEL_COMPACT;
   stats->kernel = (uint64_t)kind;
   stats->kernel_ms = ms;
   stats->tail = ctr[REBOP_CTR_SPILL];
@@ -850,6 +1100,9 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   const rebop_dev_run run_in = run; // for a rerun on the LDS kernel's int64 counts
   int rc = ensure_device();
   if (rc) return rc;
+  // a large network's kernel is free (AUTO), not asked for as REBOP_KERNEL_LDS
+  bool any_lds = kernel == REBOP_KERNEL_AUTO || kernel == kKernelAnyLds;
+  if (kernel == kKernelAnyLds) kernel = REBOP_KERNEL_LDS;
   if (kernel == REBOP_KERNEL_AUTO && g->tune_kernel >= 0 && threads == 0) {
     kernel = g->tune_kernel;
     threads = g->tune_threads;
@@ -950,13 +1203,20 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
     int width = lds_start_width(kernel, run.mode, stats != nullptr,
                                 run.x0_div ? nullptr : &g->x0);
     if (width == 2 && !compact_pays(std::vector<rebop_dev_job>{job})) width = 4;
+    IncShape shape;
+    if (any_lds && !sc && width < 8)
+      shape = inc_shape(std::vector<rebop_dev_job>{job}, g->inc_store, g->inc_depth);
     for (;;) {
       EventPair ev;
       if (stats && !sc) HIP_TRY(ev.create());
       HIP_TRY(rebop::launch_reset_counters(ctrs, stream));
       if (ev.e0) HIP_TRY(hipEventRecord(ev.e0, stream));
-      rc = enqueue_lds(std::vector<rebop_dev_job>{job}, std::vector<double>{1.0}, td, ctrs,
-                       nullptr, ctrs + REBOP_CTR_JOBQ, width, stats != nullptr, stream);
+      if (shape.ok)
+        rc = enqueue_inc(std::vector<rebop_dev_job>{job}, std::vector<double>{1.0}, shape, &g->djobs,
+                         &g->ditems, ctrs, nullptr, ctrs + REBOP_CTR_JOBQ, stats != nullptr, stream);
+      else
+        rc = enqueue_lds(std::vector<rebop_dev_job>{job}, std::vector<double>{1.0}, td, ctrs,
+                         nullptr, ctrs + REBOP_CTR_JOBQ, width, stats != nullptr, stream);
       if (rc) return rc;
       if (!stats) return REBOP_OK;
       if (ev.e1) HIP_TRY(hipEventRecord(ev.e1, stream));
@@ -964,7 +1224,8 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
       if (rc == kRetryExact) return fail(REBOP_ERR_DEVICE, "internal error: the LDS kernel flagged f64");
       if (rc != kRetryWide) return rc;
       if (width == 8) return fail(REBOP_ERR_DEVICE, "internal error: the wide LDS kernel flagged int32");
-      width *= 2;
+      width = shape.ok ? 8 : width * 2; // the incremental kernel covers int32
+      shape.ok = false;
     }
   }
   // lanes per trajectory: asked for, or (AUTO) when even 4 (2) lanes per
@@ -1507,7 +1768,7 @@ int rebop_autotune(rebop_gillespie *g, double tmax, uint64_t nb_steps, uint64_t 
     }
     if (reg_ok) cands.push_back({REBOP_KERNEL_PLAIN, threads, 1.0});
   }
-  cands.push_back({REBOP_KERNEL_LDS, 64, 1.0});
+  cands.push_back({kKernelAnyLds, 64, 1.0});
   rebop_dev_run run{};
   run.seed = g->seed;
   run.traj_begin = 0;
@@ -1537,6 +1798,7 @@ int rebop_autotune(rebop_gillespie *g, double tmax, uint64_t nb_steps, uint64_t 
     g->tune_kernel = saved;
     return fail(REBOP_ERR_UNSUPPORTED, "no kernel variant ran for this network");
   }
+  if (pick.kernel == kKernelAnyLds) pick.kernel = REBOP_KERNEL_LDS;
   g->tune_kernel = pick.kernel;
   g->tune_threads = pick.threads;
   g->tune_occ = pick.occ;
@@ -1684,6 +1946,16 @@ int rebop_run_jobs_device(const rebop_job *jobs, uint32_t n_jobs, void *stream_,
     width = std::max(width, lds_start_width(REBOP_KERNEL_AUTO, REBOP_MODE_GRID, read,
                                             jobs[j].d_x0 ? nullptr : &jobs[j].net->x0));
   if (width == 2 && !compact_pays(dj)) width = 4;
+  IncShape shape;
+  if (width < 8 && n_jobs) {
+    bool store = false;
+    uint32_t depth = 0;
+    for (uint32_t j = 0; j < n_jobs; ++j) {
+      store = store || jobs[j].net->inc_store;
+      depth = std::max(depth, jobs[j].net->inc_depth);
+    }
+    shape = inc_shape(dj, store, depth);
+  }
   rebop_stats local{};
   for (;;) {
     if (jev) HIP_TRY(rebop::launch_zero_u64(jev, n_jobs, stream));
@@ -1692,7 +1964,8 @@ int rebop_run_jobs_device(const rebop_job *jobs, uint32_t n_jobs, void *stream_,
     if (stats) HIP_TRY(ev.create());
     HIP_TRY(rebop::launch_reset_counters(ctrs, stream));
     if (ev.e0) HIP_TRY(hipEventRecord(ev.e0, stream));
-    rc = enqueue_lds(dj, cost, td, ctrs, jev, jq, width, read, stream);
+    rc = shape.ok ? enqueue_inc(dj, cost, shape, td.jobs, td.items, ctrs, jev, jq, read, stream)
+                  : enqueue_lds(dj, cost, td, ctrs, jev, jq, width, read, stream);
     if (rc) return rc;
     if (ev.e1) HIP_TRY(hipEventRecord(ev.e1, stream));
     if (!read) return REBOP_OK;
@@ -1701,7 +1974,8 @@ int rebop_run_jobs_device(const rebop_job *jobs, uint32_t n_jobs, void *stream_,
                              hipMemcpyDeviceToHost, stream));
     rc = finish_stats(&local, ctrs, ev, lds_kind(width), stream, cap_max);
     if (rc == kRetryWide && width < 8) {
-      width *= 2;
+      width = shape.ok ? 8 : width * 2;
+      shape.ok = false;
       continue;
     }
     if (rc == kRetryWide) return fail(REBOP_ERR_DEVICE, "internal error: the wide LDS kernel flagged int32");

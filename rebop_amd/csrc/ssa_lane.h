@@ -155,10 +155,12 @@ __device__ __forceinline__ uint64_t next_trajectory(const rebop_dev_run &run, bo
 
 // Whether some lane of this launch raised `flag` (a launch that will be
 // rerun: the rest of its work would be thrown away).
-__device__ __forceinline__ bool launch_stopped(const rebop_dev_run &run, uint32_t flag) {
-  return (__hip_atomic_load(&run.counters[REBOP_CTR_FLAGS], __ATOMIC_RELAXED,
-                            __HIP_MEMORY_SCOPE_AGENT) &
+__device__ __forceinline__ bool launch_flagged(const unsigned long long *counters, uint32_t flag) {
+  return (__hip_atomic_load(&counters[REBOP_CTR_FLAGS], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
           flag) != 0ull;
+}
+__device__ __forceinline__ bool launch_stopped(const rebop_dev_run &run, uint32_t flag) {
+  return launch_flagged(run.counters, flag);
 }
 
 // The draw count at which a trajectory that started this launch with d0

@@ -50,6 +50,9 @@
                                   register or specialised kernels: the host reruns such a
                                   run on the LDS kernel's int64 counts */
 
+#define REBOP_FLAG_PAST16 32u   /* a count of the incremental kernel left the int16 range (no error:
+                                  it keeps int32; the host's report of the count width reads it) */
+
 /* counters[] slots */
 #define REBOP_CTR_EVENTS 0
 #define REBOP_CTR_DRAWS 1
@@ -161,9 +164,28 @@ typedef struct {
 #define REBOP_REC_SLOW_FACTORS 0x1000u
 #define REBOP_REC_SLOW_JUMP 0x2000u
 
+/*
+ * Tables of the incremental kernel (ssa_inc.hip).  Event records, REBOP_IREC_WORDS
+ * words per reaction: its jump record (as above), then the first index and
+ * the number of the reactions its jump changes in the list inc_dep.  An entry
+ * of that list: the reaction in bits 0-15 and by how much the jump moves the
+ * counts of its first and second factor, signed, in bits 16-23 and 24-31.
+ * A reaction with a rate expression keeps, in words 0 and 1 of its reaction
+ * record, its tokens' range in inc_tok.  A token has 4 words: the operation
+ * (REBOP_OP_CONST: push) in bits 0-7 and where its last operand comes from in
+ * bits 8 and up, that operand's count row, and its constant (f64 bits, low
+ * word first): an operand read straight from a constant or a count saves the
+ * push.
+ */
+#define REBOP_IREC_WORDS 8u
+#define REBOP_TOK_STACK 0u
+#define REBOP_TOK_CONST 1u
+#define REBOP_TOK_SPECIES 2u
+
 typedef struct {
   uint32_t S, R, block, nblocks;
-  uint32_t flags, pad;
+  uint32_t flags;
+  uint32_t inc_bsh; /* log2 of the incremental kernel's block of reactions */
   const double *k;
   const uint32_t *fac_begin;
   const uint32_t *fac_s;
@@ -206,6 +228,10 @@ typedef struct {
   const uint32_t *sys_begin; /* [R+1] */
   const uint32_t *sys_species;
   const uint32_t *sys_mult;
+  /* the incremental kernel's tables (NULL: it does not run this network) */
+  const uint32_t *inc_rec; /* [R][REBOP_IREC_WORDS] */
+  const uint32_t *inc_dep;
+  const uint32_t *inc_tok; /* NULL: no rate expressions */
 } rebop_dev_job;
 
 /* a wave's unit of work: trajectories first .. first+count-1 of one job */
