@@ -69,6 +69,19 @@ typedef struct {
 #define REBOP_XOR3(a, b, c) ((a) ^ (b) ^ (c))
 #endif
 
+/* m x c as one 32 x 32 -> 64 multiply.  The compiler splits the last round's
+ * products, whose halves go different ways, into a high and a low multiply
+ * each. */
+#if defined(__HIP_DEVICE_COMPILE__) && defined(__gfx950__)
+REBOP_HD uint64_t rebop_mul32(uint32_t m, uint32_t c) {
+  uint64_t p, carry;
+  __asm__("v_mad_u64_u32 %0, %1, %2, %3, 0" : "=v"(p), "=s"(carry) : "v"(c), "s"(m));
+  return p;
+}
+#else
+REBOP_HD uint64_t rebop_mul32(uint32_t m, uint32_t c) { return (uint64_t)m * (uint64_t)c; }
+#endif
+
 /* One Philox4x32-10 block: counter (c0..c3), key (k0, k1). */
 REBOP_HD rebop_u32x4 rebop_philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                          uint32_t k0, uint32_t k1) {
@@ -76,8 +89,8 @@ REBOP_HD rebop_u32x4 rebop_philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, 
 #pragma unroll
 #endif
   for (int round = 0; round < 10; ++round) {
-    const uint64_t p0 = (uint64_t)REBOP_PHILOX_M0 * (uint64_t)c0;
-    const uint64_t p1 = (uint64_t)REBOP_PHILOX_M1 * (uint64_t)c2;
+    const uint64_t p0 = round < 9 ? (uint64_t)REBOP_PHILOX_M0 * (uint64_t)c0 : rebop_mul32(REBOP_PHILOX_M0, c0);
+    const uint64_t p1 = round < 9 ? (uint64_t)REBOP_PHILOX_M1 * (uint64_t)c2 : rebop_mul32(REBOP_PHILOX_M1, c2);
     const uint32_t hi0 = (uint32_t)(p0 >> 32), lo0 = (uint32_t)p0;
     const uint32_t hi1 = (uint32_t)(p1 >> 32), lo1 = (uint32_t)p1;
     const uint32_t n0 = REBOP_XOR3(hi1, c1, k0);
@@ -136,8 +149,8 @@ REBOP_HD rebop_u32x4 rebop_stream_block(rebop_stream s, uint64_t draw) {
   for (int round = 1; round < 10; ++round) {
     k0 += REBOP_PHILOX_W0;
     k1 += REBOP_PHILOX_W1;
-    const uint64_t q0 = (uint64_t)REBOP_PHILOX_M0 * (uint64_t)c0;
-    const uint64_t q1 = (uint64_t)REBOP_PHILOX_M1 * (uint64_t)c2;
+    const uint64_t q0 = round < 9 ? (uint64_t)REBOP_PHILOX_M0 * (uint64_t)c0 : rebop_mul32(REBOP_PHILOX_M0, c0);
+    const uint64_t q1 = round < 9 ? (uint64_t)REBOP_PHILOX_M1 * (uint64_t)c2 : rebop_mul32(REBOP_PHILOX_M1, c2);
     const uint32_t n0 = REBOP_XOR3((uint32_t)(q1 >> 32), c1, k0);
     const uint32_t n2 = REBOP_XOR3((uint32_t)(q0 >> 32), c3, k1);
     c0 = n0;
@@ -161,25 +174,37 @@ REBOP_HD rebop_u32x4 rebop_draw_block(uint64_t seed, uint64_t traj, uint64_t dra
 
 /* ---------------- uniform mappings ---------------- */
 
-/* (hi:lo >> 11) is a 53-bit integer; its conversion to double is exact. */
-REBOP_HD double rebop_u01_closed_open(uint32_t lo, uint32_t hi) {
-  const uint64_t j = ((((uint64_t)hi) << 32) | (uint64_t)lo) >> 11;
-  return (double)j * 0x1p-53;
+/* (hi:lo >> 11) is the 53-bit integer j = hi 2^21 + (lo >> 11).  Both maps
+ * are exact: hi and lo >> 11 convert exactly, and the two terms fill the 53
+ * bits of the result between them. */
+REBOP_HD double rebop_u01_closed_open(uint32_t lo, uint32_t hi) { /* j 2^-53 */
+  return __builtin_fma((double)hi, 0x1p-32, (double)(lo >> 11) * 0x1p-53);
 }
 
-REBOP_HD double rebop_u01_open_closed(uint32_t lo, uint32_t hi) {
-  const uint64_t j = (((((uint64_t)hi) << 32) | (uint64_t)lo) >> 11) + 1u;
-  return (double)j * 0x1p-53;
+REBOP_HD double rebop_u01_open_closed(uint32_t lo, uint32_t hi) { /* (j + 1) 2^-53 */
+  return __builtin_fma((double)hi, 0x1p-32, __builtin_fma((double)(lo >> 11), 0x1p-53, 0x1p-53));
 }
 
 /* ---------------- ln64 ---------------- */
 
 #define REBOP_LN2_HI 0x1.62e42ff000000p-1
 #define REBOP_LN2_LO (-0x1.718432a1b0e26p-35)
-/* bit pattern of 0.70703125, the lower end of the reduced range */
-#define REBOP_LN_BASE 0x3FE6A00000000000ull
-/* mantissa field above which m is halved (m >= 1.4140625) */
-#define REBOP_LN_HALVE 0x6a00000000000ull
+/* high word of 0.70703125, the lower end of the reduced range */
+#define REBOP_LN_BASE 0x3FE6A000u
+
+/* fma(a, b, k) for a constant k.  In device code the constant is read from
+ * scalar registers: left alone the compiler keeps the coefficients of a
+ * Horner chain in vector registers and copies each before accumulating onto
+ * it. */
+#if defined(__HIP_DEVICE_COMPILE__) && defined(__gfx950__)
+REBOP_HD double rebop_fma_k(double a, double b, double k) {
+  double d;
+  __asm__("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(k));
+  return d;
+}
+#else
+REBOP_HD double rebop_fma_k(double a, double b, double k) { return __builtin_fma(a, b, k); }
+#endif
 
 REBOP_HD uint64_t rebop_f64_bits(double x) {
   uint64_t u;
@@ -344,39 +369,35 @@ typedef struct {
   double t0, t1, t2;  /* the bucket's table row */
 } rebop_ln_pre;
 
+/* With t the high word of x less that of the range's lower end: t's
+ * arithmetic shift by 20 is k, its next seven bits the bucket, and taking its
+ * exponent field off x leaves m. */
 REBOP_HD rebop_ln_pre rebop_ln64_begin(double x, const double (*tab)[4]) {
   const uint64_t u = rebop_f64_bits(x);
-  int32_t k = (int32_t)(u >> 52) - 1023;
-  const uint64_t mant = u & 0x000fffffffffffffull;
-  uint64_t mexp = 0x3ff0000000000000ull;
-  if (mant >= REBOP_LN_HALVE) { /* m in [1.4140625, 2): use m/2, k+1 */
-    mexp = 0x3fe0000000000000ull;
-    k += 1;
-  }
-  const uint64_t mb = mexp | mant;
-  const double *t = tab[(uint32_t)((mb - REBOP_LN_BASE) >> 45)];
+  const uint32_t h = (uint32_t)(u >> 32), t = h - REBOP_LN_BASE;
+  const double *row = tab[(t >> 13) & 127u];
   rebop_ln_pre p;
-  p.m = rebop_f64_from_bits(mb);
-  p.dk = (double)k;
-  p.t0 = t[0];
-  p.t1 = t[1];
-  p.t2 = t[2];
+  p.m = rebop_f64_from_bits(((uint64_t)(h - (t & 0xfff00000u)) << 32) | (uint32_t)u);
+  p.dk = (double)((int32_t)t >> 20);
+  p.t0 = row[0];
+  p.t1 = row[1];
+  p.t2 = row[2];
   return p;
 }
 
 REBOP_HD double rebop_ln64_finish(rebop_ln_pre q) {
   const double r = __builtin_fma(q.m, q.t0, -1.0);
-  double p = -0x1p-3;                            /* -1/8 */
-  p = __builtin_fma(p, r, 0x1.2492492492492p-3);  /*  1/7 */
-  p = __builtin_fma(p, r, -0x1.5555555555555p-3); /* -1/6 */
-  p = __builtin_fma(p, r, 0x1.999999999999ap-3);  /*  1/5 */
-  p = __builtin_fma(p, r, -0x1p-2);               /* -1/4 */
-  p = __builtin_fma(p, r, 0x1.5555555555555p-2);  /*  1/3 */
+  double p = rebop_fma_k(r, -0x1p-3, 0x1.2492492492492p-3); /* -1/8, 1/7 */
+  p = rebop_fma_k(p, r, -0x1.5555555555555p-3);             /* -1/6 */
+  p = rebop_fma_k(p, r, 0x1.999999999999ap-3);              /*  1/5 */
+  p = rebop_fma_k(p, r, -0x1p-2);                           /* -1/4 */
+  p = rebop_fma_k(p, r, 0x1.5555555555555p-2);              /*  1/3 */
   const double r2 = r * r;
   const double dk = q.dk;
-  const double a = dk * REBOP_LN2_HI; /* exact: 32-bit ln2_hi times |k| <= 1075 */
-  const double hi = a + q.t1;         /* |a| >= |t1| or a == 0: Fast2Sum */
-  const double err = (a - hi) + q.t1;
+  /* k ln2_hi is exact (32 bits times |k| <= 1075), so these are Fast2Sum of
+   * it and t1 (|k ln2_hi| >= |t1| or zero) with the product inside the fma */
+  const double hi = __builtin_fma(dk, REBOP_LN2_HI, q.t1);
+  const double err = __builtin_fma(dk, REBOP_LN2_HI, -hi) + q.t1;
   const double lo = __builtin_fma(dk, REBOP_LN2_LO, q.t2) + err;
   const double tail = __builtin_fma(r2, __builtin_fma(r, p, -0.5), lo);
   return hi + (r + tail);

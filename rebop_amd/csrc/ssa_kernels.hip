@@ -33,6 +33,7 @@ struct GenericNet {
   }
 
   // the network's constants, or (parameter sweeps) this trajectory's row
+  __device__ __forceinline__ const rebop_dev_run &cold_run(const rebop_dev_run &run) const { return run; }
   __device__ __forceinline__ void start(const rebop_dev_run &run, uint64_t j) {
     const double *src = run.rates ? run.rates + (j / run.rates_div) * net.R : net.k;
 #pragma unroll

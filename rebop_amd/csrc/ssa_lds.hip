@@ -126,6 +126,7 @@ struct LdsNet {
 
   __device__ __forceinline__ uint32_t S() const { return nS; }
   __device__ __forceinline__ void start(const rebop_dev_run &, uint64_t) {}
+  __device__ __forceinline__ const rebop_dev_run &cold_run(const rebop_dev_run &run) const { return run; }
   // each job has its own horizon: computed, not tabled
   __device__ __forceinline__ double grid_time(const rebop_dev_run &run, uint64_t i) const {
     return rebop::grid_time(run, i);
