@@ -729,36 +729,134 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(int M, const __bf16 *__r
 // ---- special functions (FP64): recurrence to z >= 10, then the asymptotic
 // series of ln Gamma (Stirling) and of the digamma function, with the
 // Bernoulli-number coefficients B_2n / (2n (2n-1)) and B_2n / (2n).
-__device__ __forceinline__ double lgamma_pos(double z) {
-  // ln Gamma(z) = ln Gamma(z + n) - ln(z (z+1) ... (z+n-1)); one log of the
-  // product (at most 10 factors below 10: no overflow)
-  double prod = 1.0;
+
+// 1 / z within an ulp, for normal z away from the ends of the range
+__device__ __forceinline__ double rcp_pos(double z) {
+  double y = __builtin_amdgcn_rcp(z);
+  y = __builtin_fma(y, __builtin_fma(-z, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-z, y, 1.0), y);
+}
+
+// ln x, within an ulp, for positive normal x: x = 2^k m, m in [sqrt(1/2),
+// sqrt(2)), f = m - 1, s = f / (2 + f) and ln m = 2 atanh s = f - s (f - P),
+// P = sum 2 s^2n / (2n + 1), whose terms past n = 10 are below 2^-60 of it.
+// A third of the instructions of the library's logarithm, which carries a
+// double pair.
+__device__ __forceinline__ double ln_pos(double x) {
+  double m = __builtin_amdgcn_frexp_mant(x);
+  int k = __builtin_amdgcn_frexp_exp(x);
+  const bool low = m < 0.70710678118654752440;
+  m = low ? m + m : m;
+  k -= low ? 1 : 0;
+  const double f = m - 1.0, s = f * rcp_pos(2.0 + f), w = s * s;
+  double p = 2.0 / 21.0;
+#pragma unroll
+  for (int n = 9; n >= 1; --n) p = __builtin_fma(p, w, 2.0 / (2 * n + 1));
+  const double kd = (double)k;
+  // k ln2_hi is exact (ln2_hi has 32 bits)
+  return __builtin_fma(kd, 0x1.62e42feep-1, f - (s * (f - p * w) - kd * 0x1.a39ef35793c76p-33));
+}
+
+// ln Gamma(z) and, with PSI, digamma(z) of one z > 0: they share the
+// logarithm and the reciprocal.  With p(z) = z (z+1) ... (z+n-1),
+// ln Gamma(z) = ln Gamma(z + n) - ln p(z) and psi(z) = psi(z + n) -
+// p'(z) / p(z): one division for the whole shift (at most 10 factors below
+// 10: no overflow), and neither it nor ln p where no lane needs a shift.
+template <bool PSI>
+__device__ __forceinline__ double lgamma_digamma_pos(double z, double *psi) {
+  double prod = 1.0, dprod = 0.0;
+  const bool shifted = z < 10.0;
   while (z < 10.0) {
+    if (PSI) dprod = __builtin_fma(dprod, z, prod);
     prod *= z;
     z += 1.0;
   }
-  const double shift = log(prod);
-  const double iz = 1.0 / z, iz2 = iz * iz;
+  double shift = 0.0, dshift = 0.0;
+  if (shifted) {
+    if (prod > 0.0) {
+      shift = ln_pos(prod);
+      if (PSI) dshift = dprod * rcp_pos(prod);
+    } else { // z <= 0
+      shift = log(prod);
+      if (PSI) dshift = dprod / prod;
+    }
+  }
+  const double iz = rcp_pos(z), iz2 = iz * iz, lz = ln_pos(z);
   const double series =
       iz * (1.0 / 12.0 - iz2 * (1.0 / 360.0 - iz2 * (1.0 / 1260.0 - iz2 * (1.0 / 1680.0 - iz2 * (1.0 / 1188.0)))));
-  return (z - 0.5) * log(z) - z + 0.91893853320467274178 + series - shift;
+  if (PSI) {
+    const double dseries =
+        iz2 * (1.0 / 12.0 - iz2 * (1.0 / 120.0 - iz2 * (1.0 / 252.0 - iz2 * (1.0 / 240.0 - iz2 * (1.0 / 132.0)))));
+    *psi = lz - 0.5 * iz - dseries - dshift;
+  }
+  return (z - 0.5) * lz - z + 0.91893853320467274178 + series - shift;
+}
+__device__ __forceinline__ double lgamma_pos(double z) { return lgamma_digamma_pos<false>(z, nullptr); }
+
+// v + (v of the lane CTRL pairs this one with), a DPP rotation of a row of 16
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double v) {
+  int w[2];
+  __builtin_memcpy(w, &v, 8);
+  w[0] = __builtin_amdgcn_mov_dpp(w[0], CTRL, 0xF, 0xF, false);
+  w[1] = __builtin_amdgcn_mov_dpp(w[1], CTRL, 0xF, 0xF, false);
+  double o;
+  __builtin_memcpy(&o, w, 8);
+  return v + o;
+}
+__device__ __forceinline__ double row_sum(double v) { // over a row of 16 lanes, on every lane
+  v = dpp_add<0x128>(v); // row_ror:8
+  v = dpp_add<0x124>(v);
+  v = dpp_add<0x122>(v);
+  return dpp_add<0x121>(v);
+}
+// Two sums over pairs of lanes in one: the result is a + (a of the other half
+// of the wave) in lanes 0..31 and the same of b in lanes 32..63.
+__device__ __forceinline__ double fold32(double a, double b) {
+  uint32_t x[2], y[2];
+  __builtin_memcpy(x, &a, 8);
+  __builtin_memcpy(y, &b, 8);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+    x[i] = r[0];
+    y[i] = r[1];
+  }
+  __builtin_memcpy(&a, x, 8);
+  __builtin_memcpy(&b, y, 8);
+  return a + b;
+}
+// The same within each half: a's sum in rows 0 and 2, b's in rows 1 and 3.
+__device__ __forceinline__ double fold16(double a, double b) {
+  uint32_t x[2], y[2];
+  __builtin_memcpy(x, &a, 8);
+  __builtin_memcpy(y, &b, 8);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const auto r = __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+    x[i] = r[0];
+    y[i] = r[1];
+  }
+  __builtin_memcpy(&a, x, 8);
+  __builtin_memcpy(&b, y, 8);
+  return a + b;
 }
 
-__device__ __forceinline__ double digamma_pos(double z) {
-  double shift = 0.0;
-  while (z < 10.0) {
-    shift += 1.0 / z;
-    z += 1.0;
-  }
-  const double iz = 1.0 / z, iz2 = iz * iz;
-  const double series =
-      iz2 * (1.0 / 12.0 - iz2 * (1.0 / 120.0 - iz2 * (1.0 / 252.0 - iz2 * (1.0 / 240.0 - iz2 * (1.0 / 132.0)))));
-  return log(z) - 0.5 * iz - series - shift;
-}
+// What a mixture component's terms need besides the sample, in FP64.
+struct NllComp {
+  double lpi, pi;    // log softmax of the logits, and the softmax
+  double r, mu;      // negative binomial: dispersion and mean; binomial: mu = p
+  double lgr, psir;  // ln Gamma(r), digamma(r)
+  double c0, cx;     // ll = ... + c0 + x cx (negative binomial)
+  double spn, spp;   // softplus(-theta), softplus(theta) (binomial)
+  double irm;        // 1 / (r + mu)
+  uint32_t clamped;  // bit 0: log mean (or theta), bit 1: log dispersion
+};
 
 // Negative log-likelihood of the SSA samples under the predicted mixtures,
-// and its gradient w.r.t. the head outputs.  One wave per item, one sample
-// per lane (64 samples).  Head layout per species s (K components):
+// and its gradient w.r.t. the head outputs.  A workgroup of four waves per
+// item, one species per wave and one sample per lane (64 samples).  Head
+// layout per species s (K components):
 // [s*3K + c] mixture logit, [s*3K + K + c] log mean, [s*3K + 2K + c] log
 // dispersion.  With bounds, components c < K/2 are negative binomials of the
 // count x with log means relative to ln bound, and components c >= K/2 are
@@ -768,100 +866,163 @@ __device__ __forceinline__ double digamma_pos(double z) {
 // [nb+1][S][P * J], item (p, i) reads samples[(i*S + s) * P*J + p*J + j].
 // grad = d(mean NLL over items and samples)/d head (FP32, [B][ldh]);
 // loss_sum += total NLL (FP64).
-template <int K>
-__global__ void __launch_bounds__(64) nb_mixture_nll_kernel(
+//
+// Bound by FP64 issue.  What does not depend on the sample is computed once
+// per (species, component), one lane each, and read back from LDS; per sample
+// and negative binomial the ln Gamma and digamma share their logarithm,
+// reciprocal and shift; the responsibilities come from the exponentials of
+// the log-sum-exp; and the 64-lane sums of the 20 (unbounded: 24) gradient
+// terms halve the number of values per step instead of reducing each alone.
+// Four waves per SIMD (128 VGPRs, 28 bytes of spill) measured 61 us at 4096
+// items x 4 species x 64 samples, three 64 us, five 62 us (92 us unbounded),
+// the components unrolled at two 75 us; one wave per item with every term on
+// every lane 235 us, and at 64 items 9 us against 69 us.
+template <int K, bool BOUND>
+__global__ void __launch_bounds__(256, 4) nb_mixture_nll_kernel(
     int B, int S, int J, const float *__restrict__ head, int ldh,
     const uint32_t *__restrict__ item_point, const uint32_t *__restrict__ item_sample,
     const int64_t *__restrict__ samples, uint64_t n_traj_total, float *__restrict__ grad,
     double *__restrict__ loss_sum, double scale, const float *__restrict__ bound) {
+  constexpr int NBC = BOUND ? K / 2 : K; // negative-binomial components
+  __shared__ NllComp comp[4][K];
+  __shared__ double nbt[NBC][2][256]; // per sample: log weighted likelihood, its dispersion derivative
+  __shared__ double lcn[4]; // ln Gamma(bound + 1)
+  __shared__ double part[4];
   const int b = blockIdx.x;
-  const int j = threadIdx.x;
-  if (b >= B) return;
+  const int tid = threadIdx.x, wave = tid >> 6, j = tid & 63;
   const uint32_t p = item_point[b], i = item_sample[b];
   const bool active = j < J;
   double lane_loss = 0.0;
-  for (int s = 0; s < S; ++s) {
-    const float *h = head + (size_t)b * ldh + (size_t)s * 3 * K;
-    const double xs = active ? (double)samples[((size_t)i * S + s) * n_traj_total + (size_t)p * J + j] : 0.0;
-    const double bnd = bound ? (double)bound[(size_t)b * S + s] : 0.0;
-    const double off = bound ? log(bnd) : 0.0;
-    // log softmax of the logits (same on every lane)
-    double lmax = -1e300;
-#pragma unroll
-    for (int c = 0; c < K; ++c) lmax = fmax(lmax, (double)h[c]);
-    double zs = 0.0;
-#pragma unroll
-    for (int c = 0; c < K; ++c) zs += exp((double)h[c] - lmax);
-    const double lz = lmax + log(zs);
-    double lterm[K], mu[K], r[K], lr[K], lmu[K];
-    const double lgx1 = lgamma_pos(xs + 1.0);
-    // ln C(bound, x) for the binomial components of a bounded species
-    const double lcb = bound ? lgamma_pos(bnd + 1.0) - lgx1 - lgamma_pos(fmax(bnd - xs, 0.0) + 1.0) : 0.0;
-    double best = -1e300;
-#pragma unroll
-    for (int c = 0; c < K; ++c) {
-      double ll;
-      if (bound && c >= K / 2) {
+  for (int s0 = 0; s0 < S; s0 += 4) {
+    const int s = s0 + wave;
+    const double xs = active && s < S
+                          ? (double)samples[((size_t)i * S + s) * n_traj_total + (size_t)p * J + j]
+                          : 0.0;
+    const double bnd = BOUND && s < S ? (double)bound[(size_t)b * S + s] : 0.0;
+    // the sample-independent terms: wave 0 the components' special functions,
+    // wave 1 the softmax, wave 2 the bounds'
+    if (tid < 4 * K && s0 + tid / K < S) {
+      const int cs = tid / K, c = tid % K;
+      const float *hc = head + (size_t)b * ldh + (size_t)(s0 + cs) * 3 * K;
+      NllComp &o = comp[cs][c];
+      if (BOUND && c >= K / 2) {
         // binomial(bound, p), p = sigmoid(theta): ln p = -softplus(-theta)
-        lmu[c] = fmin(fmax((double)h[K + c], -30.0), 30.0);
-        const double th = lmu[c];
-        const double sp_neg = th < 0.0 ? log1p(exp(th)) - th : log1p(exp(-th)); // softplus(-th)
-        const double sp_pos = sp_neg + th;                                          // softplus(th)
-        mu[c] = exp(-sp_neg); // p
-        ll = lcb - xs * sp_neg - (bnd - xs) * sp_pos;
+        const double th = fmin(fmax((double)hc[K + c], -30.0), 30.0);
+        o.spn = th < 0.0 ? log1p(exp(th)) - th : log1p(exp(-th));
+        o.spp = o.spn + th;
+        o.mu = exp(-o.spn);
+        o.clamped = (double)hc[K + c] != th ? 1u : 0u;
       } else {
-        lmu[c] = fmin(fmax((double)h[K + c] + off, -8.0), 9.0);
-        lr[c] = fmin(fmax((double)h[2 * K + c], -6.0), 12.0);
-        mu[c] = exp(lmu[c]);
-        r[c] = exp(lr[c]);
-        const double lrm = log(r[c] + mu[c]);
-        ll = lgamma_pos(xs + r[c]) - lgamma_pos(r[c]) - lgx1 + r[c] * (lr[c] - lrm) +
-             xs * (lmu[c] - lrm);
+        const double off = BOUND ? log((double)bound[(size_t)b * S + s0 + cs]) : 0.0;
+        const double lm = (double)hc[K + c] + off, ld = (double)hc[2 * K + c];
+        const double lmu = fmin(fmax(lm, -8.0), 9.0), lr = fmin(fmax(ld, -6.0), 12.0);
+        const double mu = exp(lmu), r = exp(lr), lrm = log(r + mu);
+        double psi;
+        o.lgr = lgamma_digamma_pos<true>(r, &psi);
+        o.psir = psi;
+        o.mu = mu;
+        o.r = r;
+        o.c0 = r * (lr - lrm);
+        o.cx = lmu - lrm;
+        o.spn = lr - lrm;
+        o.irm = 1.0 / (r + mu);
+        o.clamped = (lm != lmu ? 1u : 0u) | (ld != lr ? 2u : 0u);
       }
-      lterm[c] = ((double)h[c] - lz) + ll;
-      best = fmax(best, lterm[c]);
+    } else if (tid >= 64 && tid < 64 + 4 * K && s0 + (tid - 64) / K < S) {
+      const int cs = (tid - 64) / K, c = (tid - 64) % K;
+      const float *hc = head + (size_t)b * ldh + (size_t)(s0 + cs) * 3 * K;
+      double lmax = -1e300, zs = 0.0;
+#pragma unroll
+      for (int q = 0; q < K; ++q) lmax = fmax(lmax, (double)hc[q]);
+#pragma unroll
+      for (int q = 0; q < K; ++q) zs += exp((double)hc[q] - lmax);
+      comp[cs][c].lpi = (double)hc[c] - (lmax + log(zs));
+      comp[cs][c].pi = exp(comp[cs][c].lpi);
+    } else if (BOUND && tid >= 128 && tid < 132 && s0 + tid - 128 < S) {
+      lcn[tid - 128] = lgamma_pos((double)bound[(size_t)b * S + s0 + tid - 128] + 1.0);
     }
-    double se = 0.0;
-#pragma unroll
-    for (int c = 0; c < K; ++c) se += exp(lterm[c] - best);
-    const double lp = best + log(se);
-    if (active) lane_loss -= lp;
-#pragma unroll
-    for (int c = 0; c < K; ++c) {
-      const double gam = active ? exp(lterm[c] - lp) : 0.0;
-      const double pi = exp((double)h[c] - lz);
-      double gl = active ? (pi - gam) : 0.0;
-      double gm, gr;
-      if (bound && c >= K / 2) {
-        gm = -gam * (xs - bnd * mu[c]); // d/dtheta of -ln binomial
-        gr = 0.0;
-        if ((double)h[K + c] != lmu[c]) gm = 0.0; // clamped
-      } else {
-        const double rm = r[c] + mu[c];
-        gm = -gam * r[c] * (xs - mu[c]) / rm;
-        gr = -gam * r[c] *
-             (digamma_pos(xs + r[c]) - digamma_pos(r[c]) + (lr[c] - log(rm)) + (mu[c] - xs) / rm);
-        if ((double)h[K + c] + off != lmu[c]) gm = 0.0; // clamped
-        if ((double)h[2 * K + c] != lr[c]) gr = 0.0;
+    __syncthreads();
+    if (s < S) { // the same for the whole wave
+      const NllComp *cp = comp[wave];
+      const double lgx1 = lgamma_pos(xs + 1.0);
+      // ln C(bound, x) for the binomial components of a bounded species
+      const double lcb = BOUND ? lcn[wave] - lgx1 - lgamma_pos(fmax(bnd - xs, 0.0) + 1.0) : 0.0;
+      // one copy of the special functions' code, its results through LDS: the
+      // registers of an unrolled loop would leave two waves per SIMD
+#pragma unroll 1
+      for (int c = 0; c < NBC; ++c) {
+        double psi;
+        const double lg = lgamma_digamma_pos<true>(xs + cp[c].r, &psi);
+        nbt[c][0][tid] = cp[c].lpi + (lg - cp[c].lgr - lgx1 + cp[c].c0 + xs * cp[c].cx);
+        nbt[c][1][tid] = psi - cp[c].psir + cp[c].spn;
       }
-      // sum over the wave's samples
+      double lterm[K];
+      double best = -1e300;
 #pragma unroll
-      for (int o = 32; o >= 1; o >>= 1) {
-        gl += __shfl_xor(gl, o);
-        gm += __shfl_xor(gm, o);
-        gr += __shfl_xor(gr, o);
+      for (int c = 0; c < K; ++c) {
+        lterm[c] = c < NBC ? nbt[c < NBC ? c : 0][0][tid]
+                           : cp[c].lpi + (lcb - xs * cp[c].spn - (bnd - xs) * cp[c].spp);
+        best = fmax(best, lterm[c]);
       }
-      if (j == 0) {
-        float *g = grad + (size_t)b * ldh + (size_t)s * 3 * K;
-        g[c] = (float)(gl * scale);
-        g[K + c] = (float)(gm * scale);
-        g[2 * K + c] = (float)(gr * scale);
+      double se = 0.0;
+#pragma unroll
+      for (int c = 0; c < K; ++c) {
+        lterm[c] = exp(lterm[c] - best);
+        se += lterm[c];
       }
+      if (active) lane_loss -= best + log(se);
+      const double ise = active ? 1.0 / se : 0.0;
+      // sums over the samples: [0, K) responsibilities, [K, 2K) log means (less
+      // a factor that is the component's), then the log dispersions
+      constexpr int NV = 2 * K + NBC;
+      static_assert(NV % 4 == 0, "folded in two halvings");
+      double v[NV];
+#pragma unroll
+      for (int c = 0; c < K; ++c) {
+        const double gam = active ? lterm[c] * ise : 0.0;
+        v[c] = gam;
+        if (c >= NBC) {
+          v[K + c] = -gam * (xs - bnd * cp[c].mu); // d/dtheta of -ln binomial
+        } else {
+          const double d = (cp[c].mu - xs) * cp[c].irm;
+          v[K + c] = gam * d;
+          v[2 * K + (c < NBC ? c : 0)] = -gam * (nbt[c < NBC ? c : 0][1][tid] + d);
+        }
+      }
+      // fold32 keeps the values below NV/2 in lanes 0..31 and the others in
+      // 32..63, fold16 halves again, and each row adds up what it is left with
+#pragma unroll
+      for (int n = 0; n < NV / 2; ++n) v[n] = fold32(v[n], v[n + NV / 2]);
+#pragma unroll
+      for (int n = 0; n < NV / 4; ++n) v[n] = row_sum(fold16(v[n], v[n + NV / 4]));
+      // row w holds the sums w NV/4 .. +NV/4 on all its lanes
+      float *g = grad + (size_t)b * ldh + (size_t)s * 3 * K;
+      double mine = 0.0;
+#pragma unroll
+      for (int n = 0; n < NV / 4; ++n)
+        if ((j & 15) == n) mine = v[n];
+      if ((j & 15) < NV / 4) {
+        const int n = (j >> 4) * (NV / 4) + (j & 15);
+        const int c = n % K;
+        if (n < K) {
+          g[n] = (float)(((double)J * cp[c].pi - mine) * scale);
+        } else if (n < 2 * K) {
+          const double f = c >= NBC ? mine : mine * cp[c].r;
+          g[n] = (float)((cp[c].clamped & 1u) ? 0.0 : f * scale);
+        } else {
+          g[n] = (float)((cp[c].clamped & 2u) ? 0.0 : mine * cp[c].r * scale);
+        }
+      }
+      if (BOUND && j < K - NBC) g[2 * K + NBC + j] = 0.f; // the binomials' unused slot
     }
+    if (s0 + 4 < S) __syncthreads(); // the components are read before the next species'
   }
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) lane_loss += __shfl_xor(lane_loss, off);
-  if (j == 0) atomicAdd(loss_sum, lane_loss);
+  lane_loss = row_sum(lane_loss);
+  lane_loss = fold16(lane_loss, lane_loss);
+  lane_loss = fold32(lane_loss, lane_loss);
+  if (j == 0) part[wave] = lane_loss;
+  __syncthreads();
+  if (tid == 0) atomicAdd(loss_sum, part[0] + part[1] + part[2] + part[3]);
 }
 
 } // namespace sg
@@ -1077,9 +1238,14 @@ int rebop_sg_nb_mixture_nll(int B, int S, int K, int J, const float *head, int l
                             const int64_t *samples, uint64_t n_traj_total, float *grad,
                             double *loss_sum, double scale, const float *bound, void *stream) {
   if (K != REBOP_SG_COMPONENTS || J > 64 || J <= 0) return 3;
-  hipLaunchKernelGGL((sg::nb_mixture_nll_kernel<REBOP_SG_COMPONENTS>), dim3(B), dim3(64), 0,
-                     (hipStream_t)stream, B, S, J, head, ldh, item_point, item_sample, samples,
-                     n_traj_total, grad, loss_sum, scale, bound);
+  if (bound)
+    hipLaunchKernelGGL((sg::nb_mixture_nll_kernel<REBOP_SG_COMPONENTS, true>), dim3(B), dim3(256), 0,
+                       (hipStream_t)stream, B, S, J, head, ldh, item_point, item_sample, samples,
+                       n_traj_total, grad, loss_sum, scale, bound);
+  else
+    hipLaunchKernelGGL((sg::nb_mixture_nll_kernel<REBOP_SG_COMPONENTS, false>), dim3(B), dim3(256), 0,
+                       (hipStream_t)stream, B, S, J, head, ldh, item_point, item_sample, samples,
+                       n_traj_total, grad, loss_sum, scale, bound);
   return ret(hipGetLastError());
 }
 

@@ -418,3 +418,49 @@ def test_trust_map_holds_on_held_out_points(sg):
     for q, xs in ssa.items():
         assert xs.shape == (sg.S, 2000)
         assert (xs[0] + xs[2] == hx[q, 0]).all()  # E + ES = E0 in every SSA sample
+
+
+@pytest.mark.parametrize("S,J,bounded", [(4, 64, True), (4, 63, False), (1, 1, True), (3, 17, False), (5, 64, True),
+                                         (9, 33, False)])
+def test_nll_kernel_species_and_samples(sg, S, J, bounded):
+    """Any number of species (four share a workgroup) and up to 64 samples,
+    with clamped parameters, counts of zero and at the bound, against the FP64
+    reference.  Terms reach ln Gamma(e^12 + x) = 1.9e6, so a sample's log
+    likelihood is good to a few ulps of that, 64 * 2^-53 * 1.9e6 = 1.3e-8, and
+    a responsibility to twice that, relative; gradients are then FP32."""
+    import torch
+
+    from oracle import surrogate_ref as ref
+
+    rng = np.random.default_rng(100 * S + J)
+    B, K, P, nb = 64, 8, 16, 4
+    ld = S * 3 * K + 8
+    bound = rng.integers(5, 2000, size=(B, S)).astype(np.float32)
+    head = rng.normal(size=(B, ld))
+    for s in range(S):
+        o = s * 3 * K
+        head[:, o + K:o + 2 * K] = rng.normal(0.0 if bounded else 4.0, 3.0, size=(B, K))
+        head[:, o + 2 * K:o + 3 * K] = rng.normal(1.0, 5.0, size=(B, K))
+    head[:, K] = 40.0  # clamped above
+    head[0, :K] = [60.0, -60.0] * 4
+    head = head.astype(np.float32)
+    ip = np.arange(B, dtype=np.int32) % P
+    isamp = (np.arange(B, dtype=np.int32) // P) + 1
+    samples = np.zeros((nb + 1, S, P * J), dtype=np.int64)
+    for b in range(B):
+        x = np.minimum(rng.integers(0, 3000, size=(S, J)) * (rng.random((S, J)) < 0.7), bound[b][:, None])
+        samples[isamp[b], :, ip[b] * J:(ip[b] + 1) * J] = x
+    dev = lambda a: torch.as_tensor(a, device="cuda")  # noqa: E731
+    d_head, d_ip, d_is, d_s, d_b = dev(head), dev(ip), dev(isamp), dev(samples), dev(bound)
+    grad = torch.zeros((B, ld), dtype=torch.float32, device="cuda")
+    loss = torch.zeros(1, dtype=torch.float64, device="cuda")
+    sg._ck(sg.load().rebop_sg_nb_mixture_nll(B, S, K, J, sg._p(d_head), ld, sg._p(d_ip), sg._p(d_is), sg._p(d_s),
+                                             P * J, sg._p(grad), sg._p(loss), 1.0,
+                                             sg._p(d_b) if bounded else None, None))
+    torch.cuda.synchronize()
+    obs = np.stack([samples[isamp[b], :, ip[b] * J:(ip[b] + 1) * J] for b in range(B)])
+    total, g = ref.nll(head.astype(np.float64), obs, K, bound=bound.astype(np.float64) if bounded else None)
+    assert abs(loss.item() - total) <= B * S * J * 1.3e-8 + 1e-12 * abs(total)
+    got = grad.double().cpu().numpy()
+    assert np.allclose(got[:, :S * 3 * K], g[:, :S * 3 * K], rtol=1e-6, atol=1e-6 * np.abs(g).max())
+    assert (got[:, S * 3 * K:] == 0).all()
