@@ -48,6 +48,32 @@ int rebop_sg_gemm_bias_act_bf16(int tb, int M, int N, int K, const void *A, int 
                                 int ldb, const float *bias, int relu, void *H, int ldh, float *F,
                                 int ldf, void *stream);
 
+/* The forward pass of a training step: layer l maps width dims[l] to
+ * dims[l+1] with the transposed weights Wt[l] [dims[l+1]][dims[l]] (BF16) and
+ * bias[l]; H[l] (l < depth - 1) receives the hidden activations
+ * [B][dims[l+1]] (BF16, after ReLU) and head the last layer's FP32 result
+ * [B][dims[depth]].  The values of rebop_sg_gemm_bias_act_bf16 layer by layer.
+ * B and all widths multiples of 64.  dims, Wt, bias and H are host arrays. */
+int rebop_sg_mlp_train_forward(int B, const void *X, int ldx, int depth, const int *dims,
+                               const void *const *Wt, const float *const *bias, void *const *H,
+                               float *head, void *stream);
+
+/* Bytes of the workspace of rebop_sg_mlp_backward (0: a shape it refuses). */
+size_t rebop_sg_mlp_backward_workspace(int B, int depth, const int *dims);
+
+/* The backward pass from d loss / d head (dhead [B][ldd], FP32) and the
+ * activations of rebop_sg_mlp_train_forward, with the weights Wb[l]
+ * [dims[l]][dims[l+1]] (BF16; Wb[0] is not read): grads receives every
+ * layer's weight gradient [dims[l]][dims[l+1]] one after the other, then
+ * every layer's bias gradient (FP32).  Gradients between layers are FP32
+ * until ReLU's derivative is applied, then BF16; bias gradients are summed
+ * from the FP32 values.  Sums are taken in a fixed order: the same inputs
+ * give the same bits.  H, Wb, workspace and grads 16-byte aligned, ldx a
+ * multiple of 8, B and all widths multiples of 64. */
+int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead, int ldd,
+                          const void *X, int ldx, const void *const *H, const void *const *Wb,
+                          void *workspace, float *grads, void *stream);
+
 /* H = bf16(act(C + bias)) and/or F = act(C + bias) (either may be NULL). */
 int rebop_sg_bias_act(int M, int N, const float *C, int ldc, const float *bias, int relu, void *H,
                       int ldh, float *F, int ldf, void *stream);

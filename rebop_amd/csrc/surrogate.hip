@@ -17,6 +17,9 @@
 
 #include <stdint.h>
 
+#include <type_traits>
+#include <vector>
+
 #include "../../include/rebop_surrogate.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -42,7 +45,12 @@ struct Epilogue {
   int ldh;
   float *F;
   int ldf;
+  bool wide;          // (gemm_nt_kernel) H and F may be written four columns at a time
+  const __bf16 *mask; // (EPI_MASK) M x N activations, lead dimension ldh
+  float *colsum;      // (EPI_MASK) [M / 64][ldc]: the column sums of each 64 rows
+  int ldc;
 };
+enum { EPI_PLAIN, EPI_BIAS, EPI_MASK };
 
 template <bool TA, bool TB, int TM, int TN, bool FUSED>
 __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const __bf16 *__restrict__ A,
@@ -123,22 +131,66 @@ __global__ void __launch_bounds__(256) gemm_kernel(int M, int N, int K, const __
       }
 }
 
+// v + (v of the lane CTRL pairs this one with), a DPP rotation of a row of 16
+template <int CTRL>
+__device__ __forceinline__ float dpp_addf(float v) {
+  int w;
+  __builtin_memcpy(&w, &v, 4);
+  w = __builtin_amdgcn_mov_dpp(w, CTRL, 0xF, 0xF, false);
+  float o;
+  __builtin_memcpy(&o, &w, 4);
+  return v + o;
+}
+__device__ __forceinline__ float row_sumf(float v) { // over a row of 16 lanes, on every lane
+  v = dpp_addf<0x128>(v); // row_ror:8
+  v = dpp_addf<0x124>(v);
+  v = dpp_addf<0x122>(v);
+  return dpp_addf<0x121>(v);
+}
+
+// The tile of this workgroup.  Consecutive workgroups go to different XCDs;
+// taken in linear order the eight tiles of one block of rows would be read
+// through eight L2 caches.  XCD x gets the x-th eighth of the tiles instead,
+// so it reads its own rows of A (the rows it wrote in the layer before) and
+// all of B.
+__device__ __forceinline__ void xcd_tile(int &bx, int &by) {
+  const int gx = (int)gridDim.x, total = gx * (int)gridDim.y;
+  bx = (int)blockIdx.x;
+  by = (int)blockIdx.y;
+  if (total % 8 == 0) {
+    const int lin = bx + gx * by, t = (lin & 7) * (total >> 3) + (lin >> 3);
+    bx = t % gx;
+    by = t / gx;
+  }
+}
+
 // The same product for A [M][K] and B stored [N][K] (both k-contiguous, as
-// the forward pass and the backward's dX use them), software-pipelined: the
-// next 32-wide k slice is loaded from global memory into registers while the
-// matrix cores work on the current one, which sits in one of two LDS
-// buffers, so one barrier per slice separates the stores into the other
-// buffer from its reads.  Same tiles, fragments and summation order per
-// output as gemm_kernel<false, true>.
-template <int TM, int TN, bool FUSED>
+// the forward pass and the backward's dX use them).  Bound by the latency of
+// its loads: a slice's MFMAs take a fraction of the time its loads need to
+// arrive, so two 64-wide slices are under way in registers while a third is
+// multiplied out of one of two LDS buffers, with one barrier per slice.  The
+// MFMA of the fused epilogues takes B's rows as its first operand, so that a
+// lane's four outputs are four consecutive columns of one row, written at
+// once.  Same products and summation order per output as
+// gemm_kernel<false, true>.
+// EPI_BIAS: act(C + bias) as in gemm_kernel.  EPI_MASK: the ReLU derivative
+// from the stored activation, epi.H = bf16(mask > 0 ? C : 0), and epi.colsum
+// the FP32 sums of its columns (the bias gradient's parts).
+// 4096 x 512 x 512: 8.4 us with bias and ReLU (one 32-wide slice ahead:
+// 10.0 us), 8.7 us with mask and column sums (8.8 us for the product, 7.5 us
+// for the mask and 20 us for the sums as passes of their own).
+template <int TM, int TN, int EPI>
 __global__ void __launch_bounds__(256) gemm_nt_kernel(int M, int N, int K, const __bf16 *__restrict__ A,
                                                       int lda, const __bf16 *__restrict__ B, int ldb,
                                                       float *__restrict__ C, int ldc, Epilogue epi) {
-  constexpr int FM = TM / 32, FN = TN / 32, PA = TM / 64, PB = TN / 64;
-  __shared__ __attribute__((aligned(16))) __bf16 As[2][TM][40];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][TN][40];
+  constexpr int FM = TM / 32, FN = TN / 32, PA = TM / 32, PB = TN / 32, BK = 64;
+  constexpr int LD = BK + 8; // 144 B: sixteen rows start in different banks
+  __shared__ __attribute__((aligned(16))) __bf16 As[2][TM][LD];
+  __shared__ __attribute__((aligned(16))) __bf16 Bs[2][TN][LD];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
+  int bx, by;
+  xcd_tile(bx, by);
+  const int m0 = by * TM, n0 = bx * TN;
   const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
   floatx4 acc[FM][FN];
 #pragma unroll
@@ -146,74 +198,305 @@ __global__ void __launch_bounds__(256) gemm_nt_kernel(int M, int N, int K, const
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  const int ksplit = K / (int)gridDim.z;
+  const int ksplit = K / (int)gridDim.z; // a multiple of 32 (checked by the host)
   const int kbeg = (int)blockIdx.z * ksplit, kend = kbeg + ksplit;
-  // thread tid moves the 8-element chunks tid + 256 p: row (chunk >> 2), k (chunk & 3) * 8
-  bf16x8 ra[PA], rb[PB];
-  auto gload = [&](int k0) {
+  const int nk = (ksplit + BK - 1) / BK;
+  // thread tid moves the 8-element chunks tid + 256 p: row (chunk >> 3), k
+  // (chunk & 7) * 8; past kend (half a slice) it stores zeros
+  const int lr = tid >> 3, lc = (tid & 7) * 8;
+  bf16x8 ra[2][PA], rb[2][PB];
+  auto gload = [&](auto set, int it) {
+    constexpr int q = decltype(set)::value;
+    const int k = kbeg + it * BK + lc;
+    const bool in = k < kend;
 #pragma unroll
-    for (int p = 0; p < PA; ++p) {
-      const int idx = tid + 256 * p, r = idx >> 2, c = (idx & 3) * 8;
-      ra[p] = *(const bf16x8 *)&A[(size_t)(m0 + r) * lda + k0 + c];
-    }
+    for (int p = 0; p < PA; ++p)
+      ra[q][p] = in ? *(const bf16x8 *)&A[(size_t)(m0 + lr + 32 * p) * lda + k] : bf16x8{};
 #pragma unroll
-    for (int p = 0; p < PB; ++p) {
-      const int idx = tid + 256 * p, r = idx >> 2, c = (idx & 3) * 8;
-      rb[p] = *(const bf16x8 *)&B[(size_t)(n0 + r) * ldb + k0 + c];
-    }
+    for (int p = 0; p < PB; ++p)
+      rb[q][p] = in ? *(const bf16x8 *)&B[(size_t)(n0 + lr + 32 * p) * ldb + k] : bf16x8{};
   };
-  auto lstore = [&](int buf) {
+  auto lstore = [&](auto set) { // register set q goes to LDS buffer q
+    constexpr int q = decltype(set)::value;
 #pragma unroll
-    for (int p = 0; p < PA; ++p) {
-      const int idx = tid + 256 * p, r = idx >> 2, c = (idx & 3) * 8;
-      *(bf16x8 *)&As[buf][r][c] = ra[p];
-    }
+    for (int p = 0; p < PA; ++p) *(bf16x8 *)&As[q][lr + 32 * p][lc] = ra[q][p];
 #pragma unroll
-    for (int p = 0; p < PB; ++p) {
-      const int idx = tid + 256 * p, r = idx >> 2, c = (idx & 3) * 8;
-      *(bf16x8 *)&Bs[buf][r][c] = rb[p];
-    }
+    for (int p = 0; p < PB; ++p) *(bf16x8 *)&Bs[q][lr + 32 * p][lc] = rb[q][p];
   };
-  gload(kbeg);
-  lstore(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += 32) {
-    const bool more = k0 + 32 < kend;
-    if (more) gload(k0 + 32); // in flight during the MFMAs below
-    bf16x8 a[FM], b[FN];
+  typedef std::integral_constant<int, 0> set0;
+  typedef std::integral_constant<int, 1> set1;
+  auto step = [&](auto set, auto other, int it) {
+    constexpr int q = decltype(set)::value;
+    if (it + 2 < nk) gload(set, it + 2);
 #pragma unroll
-    for (int i = 0; i < FM; ++i) a[i] = *(const bf16x8 *)&As[buf][wm + i * 16 + (lane & 15)][(lane >> 4) * 8];
+    for (int kk = 0; kk < BK; kk += 32) {
+      bf16x8 a[FM], b[FN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) b[j] = *(const bf16x8 *)&Bs[buf][wn + j * 16 + (lane & 15)][(lane >> 4) * 8];
+      for (int i = 0; i < FM; ++i) a[i] = *(const bf16x8 *)&As[q][wm + i * 16 + (lane & 15)][kk + (lane >> 4) * 8];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+      for (int j = 0; j < FN; ++j) b[j] = *(const bf16x8 *)&Bs[q][wn + j * 16 + (lane & 15)][kk + (lane >> 4) * 8];
 #pragma unroll
-      for (int j = 0; j < FN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    if (more) lstore(buf ^ 1); // that buffer's reads ended at the last barrier
+      for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+          acc[i][j] = EPI == EPI_PLAIN ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0)
+                                       : __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);
+    }
+    if (it + 1 < nk) lstore(other); // that buffer's reads ended at the last barrier
     __syncthreads();
-    buf ^= 1;
+  };
+  gload(set0{}, 0);
+  if (nk > 1) gload(set1{}, 1);
+  lstore(set0{});
+  __syncthreads();
+  for (int it = 0; it < nk; it += 2) {
+    step(set0{}, set1{}, it);
+    if (it + 1 < nk) step(set1{}, set0{}, it + 1);
   }
+
+  floatx4 cs[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) cs[j] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      if constexpr (EPI == EPI_PLAIN) {
+        const int row = m0 + wm + i * 16 + (lane >> 4) * 4, col = n0 + wn + j * 16 + (lane & 15);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float *o = &C[(size_t)(row + q) * ldc + col];
+          if (gridDim.z == 1) *o = acc[i][j][q];
+          else atomicAdd(o, acc[i][j][q]);
+        }
+      } else {
+        const int row = m0 + wm + i * 16 + (lane & 15), col = n0 + wn + j * 16 + (lane >> 4) * 4;
+        floatx4 v = acc[i][j];
+        __bf16 h[4];
+        if constexpr (EPI == EPI_MASK) {
+          __bf16 mk[4];
+          __builtin_memcpy(mk, __builtin_assume_aligned(&epi.mask[(size_t)row * epi.ldh + col], 8), sizeof mk);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) v[q] = (float)mk[q] > 0.f ? v[q] : 0.f;
+          cs[j] += v;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            v[q] += epi.bias[col + q];
+            if (epi.relu) v[q] = v[q] > 0.f ? v[q] : 0.f;
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) h[q] = (__bf16)v[q];
+        __bf16 *oh = epi.H + (size_t)row * epi.ldh + col;
+        float *of = epi.F + (size_t)row * epi.ldf + col;
+        if (EPI == EPI_MASK || epi.wide) {
+          if (epi.H) __builtin_memcpy(__builtin_assume_aligned(oh, 8), h, sizeof h);
+          if (EPI == EPI_BIAS && epi.F) *(floatx4 *)of = v;
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (epi.H) oh[q] = h[q];
+            if (epi.F) of[q] = v[q];
+          }
+        }
+      }
+    }
+  if constexpr (EPI == EPI_MASK) {
+    float(*red)[TN] = (float(*)[TN])As; // the last reads of As are behind a barrier
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int row = m0 + wm + i * 16 + (lane >> 4) * 4 + q;
-        const int col = n0 + wn + j * 16 + (lane & 15);
-        if (FUSED) {
-          float v = acc[i][j][q] + epi.bias[col];
-          if (epi.relu) v = v > 0.f ? v : 0.f;
-          if (epi.H) epi.H[(size_t)row * epi.ldh + col] = (__bf16)v;
-          if (epi.F) epi.F[(size_t)row * epi.ldf + col] = v;
-        } else if (gridDim.z == 1) {
-          C[(size_t)row * ldc + col] = acc[i][j][q];
-        } else {
-          atomicAdd(&C[(size_t)row * ldc + col], acc[i][j][q]);
-        }
+        const float t = row_sumf(cs[j][q]);
+        if ((lane & 15) == 0) red[wave >> 1][wn + j * 16 + (lane >> 4) * 4 + q] = t;
       }
+    __syncthreads();
+    // a wave covers TM / 2 rows
+    if (tid < TN) {
+      float *o = epi.colsum + (size_t)by * (TM / 64) * epi.ldc + n0 + tid;
+      if constexpr (TM == 64) {
+        *o = red[0][tid] + red[1][tid];
+      } else {
+        o[0] = red[0][tid];
+        o[epi.ldc] = red[1][tid];
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// The weight gradients of every layer in one launch: dW_l = H_l^T dZ_l, H_l
+// [B][m_l] and dZ_l [B][n_l] both with the contraction index b outermost.
+// A workgroup takes a 64 x 64 tile of one layer and a range of the batch
+// (split z of gridDim.y), 64 rows at a time: a thread reads 8 columns of 4
+// rows, transposes them with byte permutes, and writes 4 consecutive b of
+// each column to LDS, from where the MFMA fragments are read.  The rows after
+// the current ones are on their way in registers meanwhile.  A layer at a
+// time would leave the chip a quarter full; all of them give 216 tiles (five
+// layers, width 512).  Splits write their sums to part[z], which
+// grad_reduce_kernel adds in order: no atomics, and the same bits every run.
+constexpr int WG_MAXL = 8;
+struct WgradNet {
+  const __bf16 *H[WG_MAXL], *dZ[WG_MAXL];
+  int n[WG_MAXL]; // multiples of 64, as the widths of H
+  int ldh[WG_MAXL];
+  int tile0[WG_MAXL];       // first tile of layer l
+  size_t out[WG_MAXL];      // where dW_l starts, in floats
+  int layers;
+};
+
+__global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, float *__restrict__ part,
+                                                    size_t stride) {
+  constexpr int LD = 68; // 136 B rows: 8-byte accesses, at most two lanes per bank
+  __shared__ __attribute__((aligned(16))) __bf16 T[2][2][64][LD]; // [buffer][H, dZ][column][b]
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const __bf16 *H = net.H[0], *Z = net.dZ[0];
+  int n = net.n[0], ldh = net.ldh[0], t0 = 0;
+  size_t out = net.out[0];
+#pragma unroll
+  for (int l = 1; l < WG_MAXL; ++l)
+    if (l < net.layers && (int)blockIdx.x >= net.tile0[l]) {
+      H = net.H[l];
+      Z = net.dZ[l];
+      n = net.n[l];
+      ldh = net.ldh[l];
+      t0 = net.tile0[l];
+      out = net.out[l];
+    }
+  const int t = (int)blockIdx.x - t0, tn = n / 64, m0 = t / tn * 64, n0 = t % tn * 64;
+  const int ubeg = (int)((int64_t)units * blockIdx.y / gridDim.y);
+  const int uend = (int)((int64_t)units * (blockIdx.y + 1) / gridDim.y);
+  const int side = tid >> 7, cg = tid & 7, kq = (tid & 127) >> 3;
+  const size_t ld = side ? (size_t)n : (size_t)ldh;
+  const __bf16 *src = (side ? Z + n0 : H + m0) + (size_t)(4 * kq) * ld + 8 * cg;
+  uint32_t r[4][4];
+  auto gload = [&](int u) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint4 v = *(const uint4 *)(src + ((size_t)u * 64 + i) * ld);
+      r[i][0] = v.x;
+      r[i][1] = v.y;
+      r[i][2] = v.z;
+      r[i][3] = v.w;
+    }
+  };
+  auto lstore = [&](int buf) {
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      uint2 lo, hi; // columns 2 w and 2 w + 1, rows 0..3
+      lo.x = __builtin_amdgcn_perm(r[1][w], r[0][w], 0x05040100u);
+      lo.y = __builtin_amdgcn_perm(r[3][w], r[2][w], 0x05040100u);
+      hi.x = __builtin_amdgcn_perm(r[1][w], r[0][w], 0x07060302u);
+      hi.y = __builtin_amdgcn_perm(r[3][w], r[2][w], 0x07060302u);
+      *(uint2 *)&T[buf][side][8 * cg + 2 * w][4 * kq] = lo;
+      *(uint2 *)&T[buf][side][8 * cg + 2 * w + 1][4 * kq] = hi;
+    }
+  };
+  auto frag = [&](int buf, int s, int c, int k) { // 8 consecutive b of column c
+    bf16x8 v;
+    uint2 a[2];
+    a[0] = *(const uint2 *)&T[buf][s][c][k];
+    a[1] = *(const uint2 *)&T[buf][s][c][k + 4];
+    __builtin_memcpy(&v, a, sizeof v);
+    return v;
+  };
+  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  floatx4 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  gload(ubeg);
+  lstore(0);
+  __syncthreads();
+  int buf = 0;
+  for (int u = ubeg; u < uend; ++u) {
+    if (u + 1 < uend) gload(u + 1);
+#pragma unroll
+    for (int kk = 0; kk < 64; kk += 32) {
+      bf16x8 h[2], z[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) h[i] = frag(buf, 0, wm + i * 16 + (lane & 15), kk + (lane >> 4) * 8);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) z[j] = frag(buf, 1, wn + j * 16 + (lane & 15), kk + (lane >> 4) * 8);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(z[j], h[i], acc[i][j], 0, 0, 0);
+    }
+    if (u + 1 < uend) lstore(buf ^ 1); // that buffer's reads ended at the last barrier
+    __syncthreads();
+    buf ^= 1;
+  }
+  float *o = part + stride * blockIdx.y + out;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = m0 + wm + i * 16 + (lane & 15), col = n0 + wn + j * 16 + (lane >> 4) * 4;
+      *(floatx4 *)&o[(size_t)row * n + col] = acc[i][j];
+    }
+}
+
+// The head's gradient as the backward pass reads it: dZ = bf16(g) and the
+// column sums of each 64 rows, 64 x 64 per workgroup.
+__global__ void __launch_bounds__(256) head_grad_kernel(int N, const float *__restrict__ g, int ldg,
+                                                        __bf16 *__restrict__ dZ, float *__restrict__ colsum,
+                                                        int ldc) {
+  __shared__ float red[16][64];
+  const int c4 = (threadIdx.x & 15) * 4, rg = threadIdx.x >> 4;
+  const int n = blockIdx.x * 64 + c4;
+  float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const size_t row = (size_t)blockIdx.y * 64 + rg + 16 * i;
+    __bf16 h[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float v = g[row * ldg + n + q];
+      s[q] += v;
+      h[q] = (__bf16)v;
+    }
+    __builtin_memcpy(&dZ[row * N + n], h, sizeof h);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) red[rg][c4 + q] = s[q];
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += red[i][threadIdx.x];
+    colsum[(size_t)blockIdx.y * ldc + blockIdx.x * 64 + threadIdx.x] = t;
+  }
+}
+
+// grads[0, weights) = the sum of the splits' parts (splits > 1: else they are
+// in place), 1024 floats per workgroup; then the bias gradients, 64 per
+// workgroup, from the column sums [rows][nbias] of every layer side by side.
+__global__ void __launch_bounds__(256) grad_reduce_kernel(int splits, size_t weights, size_t stride,
+                                                          const float *__restrict__ part, int nbias,
+                                                          int rows, const float *__restrict__ colsum,
+                                                          float *__restrict__ grads) {
+  const unsigned wblk = splits > 1 ? (unsigned)(weights / 1024) : 0u;
+  if (blockIdx.x < wblk) {
+    const size_t i = (size_t)blockIdx.x * 1024 + threadIdx.x * 4;
+    floatx4 v = *(const floatx4 *)&part[i];
+    for (int z = 1; z < splits; ++z) v += *(const floatx4 *)&part[stride * z + i];
+    *(floatx4 *)&grads[i] = v;
+    return;
+  }
+  __shared__ float red[4][64];
+  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int n = (int)(blockIdx.x - wblk) * 64 + c;
+  float s = 0.f;
+  if (n < nbias)
+#pragma unroll 8
+    for (int m = g; m < rows; m += 4) s += colsum[(size_t)m * nbias + n];
+  red[g][c] = s;
+  __syncthreads();
+  if (g == 0 && n < nbias) grads[weights + n] = red[0][c] + red[1][c] + red[2][c] + red[3][c];
 }
 
 __global__ void zero_kernel(int M, int N, float *__restrict__ C, int ldc) {
@@ -1057,38 +1340,84 @@ int mlp_net(int depth, const int *dims, const void *const *Wp, const float *cons
   return 0;
 }
 
-template <bool TA, bool TB>
-void launch_gemm(bool big, dim3 grid, hipStream_t s, int M, int N, int K, const __bf16 *a,
-                        int lda, const __bf16 *b, int ldb, float *C, int ldc,
-                        const sg::Epilogue *epi = nullptr) {
-  const sg::Epilogue none{nullptr, 0, nullptr, 0, nullptr, 0};
-  if (!TA && TB) { // k-contiguous operands: the pipelined kernel
-    if (big && epi)
-      hipLaunchKernelGGL((sg::gemm_nt_kernel<128, 128, true>), grid, dim3(256), 0, s, M, N, K, a, lda,
-                         b, ldb, C, ldc, *epi);
-    else if (epi)
-      hipLaunchKernelGGL((sg::gemm_nt_kernel<64, 64, true>), grid, dim3(256), 0, s, M, N, K, a, lda,
-                         b, ldb, C, ldc, *epi);
-    else if (big)
-      hipLaunchKernelGGL((sg::gemm_nt_kernel<128, 128, false>), grid, dim3(256), 0, s, M, N, K, a,
-                         lda, b, ldb, C, ldc, none);
-    else
-      hipLaunchKernelGGL((sg::gemm_nt_kernel<64, 64, false>), grid, dim3(256), 0, s, M, N, K, a, lda,
-                         b, ldb, C, ldc, none);
-    return;
-  }
-  if (epi && big)
-    hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 128, 128, true>), grid, dim3(256), 0, s, M, N, K, a,
-                       lda, b, ldb, C, ldc, *epi);
-  else if (epi)
-    hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 64, 64, true>), grid, dim3(256), 0, s, M, N, K, a,
-                       lda, b, ldb, C, ldc, *epi);
-  else if (big)
-    hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 128, 128, false>), grid, dim3(256), 0, s, M, N, K, a,
-                       lda, b, ldb, C, ldc, none);
+// 128 x 128 tiles when there are enough of them to fill the chip
+bool big_tiles(int M, int N) { return M % 128 == 0 && N % 128 == 0 && (M / 128) * (N / 128) >= 512; }
+
+// k-contiguous operands: the pipelined kernel
+template <int EPI>
+void launch_nt(bool big, dim3 grid, hipStream_t s, int M, int N, int K, const __bf16 *a, int lda,
+               const __bf16 *b, int ldb, float *C, int ldc, const sg::Epilogue &epi) {
+  if (big)
+    hipLaunchKernelGGL((sg::gemm_nt_kernel<128, 128, EPI>), grid, dim3(256), 0, s, M, N, K, a, lda, b, ldb, C,
+                       ldc, epi);
   else
-    hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 64, 64, false>), grid, dim3(256), 0, s, M, N, K, a,
-                       lda, b, ldb, C, ldc, none);
+    hipLaunchKernelGGL((sg::gemm_nt_kernel<64, 64, EPI>), grid, dim3(256), 0, s, M, N, K, a, lda, b, ldb, C,
+                       ldc, epi);
+}
+
+template <bool TA, bool TB>
+void launch_gemm(bool big, dim3 grid, hipStream_t s, int M, int N, int K, const __bf16 *a, int lda,
+                 const __bf16 *b, int ldb, float *C, int ldc, const sg::Epilogue *epi = nullptr) {
+  if constexpr (!TA && TB) {
+    if (epi) launch_nt<sg::EPI_BIAS>(big, grid, s, M, N, K, a, lda, b, ldb, C, ldc, *epi);
+    else launch_nt<sg::EPI_PLAIN>(big, grid, s, M, N, K, a, lda, b, ldb, C, ldc, sg::Epilogue{});
+    return;
+  } else {
+    const sg::Epilogue e = epi ? *epi : sg::Epilogue{};
+    if (epi && big)
+      hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 128, 128, true>), grid, dim3(256), 0, s, M, N, K, a, lda, b,
+                         ldb, C, ldc, e);
+    else if (epi)
+      hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 64, 64, true>), grid, dim3(256), 0, s, M, N, K, a, lda, b, ldb,
+                         C, ldc, e);
+    else if (big)
+      hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 128, 128, false>), grid, dim3(256), 0, s, M, N, K, a, lda, b,
+                         ldb, C, ldc, e);
+    else
+      hipLaunchKernelGGL((sg::gemm_kernel<TA, TB, 64, 64, false>), grid, dim3(256), 0, s, M, N, K, a, lda, b,
+                         ldb, C, ldc, e);
+  }
+}
+
+sg::Epilogue bias_epilogue(const float *bias, int relu, void *H, int ldh, float *F, int ldf) {
+  sg::Epilogue e{};
+  e.bias = bias;
+  e.relu = relu;
+  e.H = (__bf16 *)H;
+  e.ldh = ldh;
+  e.F = F;
+  e.ldf = ldf;
+  e.wide = (!H || ((uintptr_t)H % 8 == 0 && ldh % 4 == 0)) && (!F || ((uintptr_t)F % 16 == 0 && ldf % 4 == 0));
+  return e;
+}
+
+// The shapes of a layer stack's training passes, and how the backward pass
+// lays out its workspace: dZ of every layer (BF16), the column sums
+// [batch / 64][sum of widths], and with splits > 1 their weight gradients.
+struct TrainPlan {
+  size_t weights = 0, dz = 0, colsum = 0, part = 0; // floats; BF16 elements; floats; floats
+  int nbias = 0, splits = 1, units = 0;
+  size_t bytes() const { return 2 * dz + 4 * colsum + 4 * part; }
+};
+bool train_plan(int B, int depth, const int *dims, TrainPlan &p) {
+  if (B <= 0 || B % 64 || depth < 1 || !dims) return false;
+  size_t tiles = 0;
+  for (int l = 0; l <= depth; ++l) {
+    if (dims[l] <= 0 || dims[l] % 64) return false;
+    if (l == 0) continue;
+    p.weights += (size_t)dims[l - 1] * dims[l];
+    tiles += (size_t)(dims[l - 1] / 64) * (dims[l] / 64);
+    p.nbias += dims[l];
+  }
+  p.units = B / 64;
+  // about 1024 workgroups (four to a CU) of at least 128 rows each
+  size_t z = 1024 / tiles;
+  if (z > (size_t)p.units / 2) z = (size_t)p.units / 2;
+  p.splits = z < 1 ? 1 : z > 32 ? 32 : (int)z;
+  p.dz = (size_t)B * p.nbias;
+  p.colsum = (size_t)p.units * p.nbias;
+  p.part = p.splits > 1 ? p.weights * (size_t)p.splits : 0;
+  return true;
 }
 
 } // namespace
@@ -1100,8 +1429,7 @@ const char *rebop_sg_last_error(void) { return hipGetErrorString(g_err); }
 int rebop_sg_gemm_bf16(int ta, int tb, int M, int N, int K, const void *A, int lda, const void *B,
                        int ldb, float *C, int ldc, void *stream) {
   if (M % 64 || N % 64 || K % 32 || M <= 0 || N <= 0 || K <= 0) return 3;
-  // 128 x 128 tiles when there are enough of them to fill the chip
-  const bool big = M % 128 == 0 && N % 128 == 0 && (M / 128) * (N / 128) >= 512;
+  const bool big = big_tiles(M, N);
   const int tile = big ? 128 : 64;
   // split K when the output has too few tiles to fill the chip
   int splits = 1;
@@ -1125,16 +1453,107 @@ int rebop_sg_gemm_bias_act_bf16(int tb, int M, int N, int K, const void *A, int 
                                 int ldf, void *stream) {
   if (M % 64 || N % 64 || K % 32 || M <= 0 || N <= 0 || K <= 0) return 3;
   if (!bias || (!H && !F)) return 3;
-  const bool big = M % 128 == 0 && N % 128 == 0 && (M / 128) * (N / 128) >= 512;
+  const bool big = big_tiles(M, N);
   const int tile = big ? 128 : 64;
   const dim3 grid(N / tile, M / tile, 1); // no split K: the epilogue needs the whole sum
-  const sg::Epilogue epi{bias, relu, (__bf16 *)H, ldh, F, ldf};
+  const sg::Epilogue epi = bias_epilogue(bias, relu, H, ldh, F, ldf);
   if (tb)
     launch_gemm<false, true>(big, grid, (hipStream_t)stream, M, N, K, (const __bf16 *)A, lda,
                              (const __bf16 *)B, ldb, nullptr, 0, &epi);
   else
     launch_gemm<false, false>(big, grid, (hipStream_t)stream, M, N, K, (const __bf16 *)A, lda,
                               (const __bf16 *)B, ldb, nullptr, 0, &epi);
+  return ret(hipGetLastError());
+}
+
+int rebop_sg_mlp_train_forward(int B, const void *X, int ldx, int depth, const int *dims,
+                               const void *const *Wt, const float *const *bias, void *const *H,
+                               float *head, void *stream) {
+  TrainPlan p;
+  if (!train_plan(B, depth, dims, p) || !X || !Wt || !bias || !head || (depth > 1 && !H) || ldx < dims[0] || ldx % 8)
+    return 3;
+  for (int l = 0; l < depth; ++l)
+    if (!Wt[l] || !bias[l] || (l < depth - 1 && !H[l])) return 3;
+  const void *in = X;
+  for (int l = 0; l < depth; ++l) {
+    const bool last = l == depth - 1;
+    const int rc = rebop_sg_gemm_bias_act_bf16(1, B, dims[l + 1], dims[l], in, l == 0 ? ldx : dims[l], Wt[l],
+                                               dims[l], bias[l], !last, last ? nullptr : H[l], dims[l + 1],
+                                               last ? head : nullptr, dims[l + 1], stream);
+    if (rc) return rc;
+    if (!last) in = H[l];
+  }
+  return 0;
+}
+
+size_t rebop_sg_mlp_backward_workspace(int B, int depth, const int *dims) {
+  TrainPlan p;
+  return train_plan(B, depth, dims, p) ? p.bytes() : 0;
+}
+
+int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead, int ldd, const void *X, int ldx,
+                          const void *const *H, const void *const *Wb, void *workspace, float *grads,
+                          void *stream) {
+  TrainPlan p;
+  if (!train_plan(B, depth, dims, p) || !dhead || !X || !Wb || !workspace || !grads || (depth > 1 && !H) ||
+      ldd < dims[depth] || ldx < dims[0] || ldx % 8 || (uintptr_t)workspace % 16 ||
+      (uintptr_t)grads % 16)
+    return 3;
+  for (int l = 1; l < depth; ++l)
+    if (!H[l - 1] || !Wb[l] || (uintptr_t)H[l - 1] % 16 || (uintptr_t)Wb[l] % 16) return 3;
+  hipStream_t s = (hipStream_t)stream;
+  float *part = (float *)workspace, *colsum = part + p.part;
+  __bf16 *dz = (__bf16 *)(colsum + p.colsum); // p.part and p.colsum are multiples of 64
+  size_t dz_end = p.dz;
+  int col = p.nbias;
+  auto layer_dz = [&](int l) { return dz + dz_end - (size_t)B * dims[l + 1]; };
+  // dZ from the last layer to the first, each with its column sums
+  std::vector<const __bf16 *> dZ((size_t)depth);
+  for (int l = depth - 1; l >= 0; --l) {
+    const int n = dims[l + 1];
+    __bf16 *out = layer_dz(l);
+    col -= n;
+    if (l == depth - 1) {
+      hipLaunchKernelGGL(sg::head_grad_kernel, dim3(n / 64, B / 64), dim3(256), 0, s, n, dhead, ldd, out,
+                         colsum + col, p.nbias);
+    } else {
+      sg::Epilogue e{};
+      e.H = out;
+      e.ldh = n;
+      e.mask = (const __bf16 *)H[l];
+      e.colsum = colsum + col;
+      e.ldc = p.nbias;
+      const bool big = big_tiles(B, n);
+      const int tile = big ? 128 : 64, k = dims[l + 2];
+      launch_nt<sg::EPI_MASK>(big, dim3(n / tile, B / tile), s, B, n, k, dZ[l + 1], k, (const __bf16 *)Wb[l + 1], k,
+                              nullptr, 0, e);
+    }
+    dZ[l] = out;
+    dz_end -= (size_t)B * n;
+  }
+  // every layer's weight gradient
+  float *wout = p.splits > 1 ? part : grads;
+  size_t at = 0;
+  for (int l0 = 0; l0 < depth; l0 += sg::WG_MAXL) {
+    sg::WgradNet net{};
+    int tiles = 0;
+    for (int l = l0; l < depth && l < l0 + sg::WG_MAXL; ++l) {
+      const int i = l - l0;
+      net.H[i] = (const __bf16 *)(l == 0 ? X : H[l - 1]);
+      net.ldh[i] = l == 0 ? ldx : dims[l];
+      net.dZ[i] = dZ[l];
+      net.n[i] = dims[l + 1];
+      net.tile0[i] = tiles;
+      net.out[i] = at;
+      net.layers = i + 1;
+      tiles += (dims[l] / 64) * (dims[l + 1] / 64);
+      at += (size_t)dims[l] * dims[l + 1];
+    }
+    hipLaunchKernelGGL(sg::wgrad_kernel, dim3(tiles, p.splits), dim3(256), 0, s, p.units, net, wout, p.weights);
+  }
+  const unsigned blocks = (p.splits > 1 ? (unsigned)(p.weights / 1024) : 0u) + nblk((size_t)p.nbias, 64);
+  hipLaunchKernelGGL(sg::grad_reduce_kernel, dim3(blocks), dim3(256), 0, s, p.splits, p.weights, p.weights, part,
+                     p.nbias, p.units, colsum, grads);
   return ret(hipGetLastError());
 }
 

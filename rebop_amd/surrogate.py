@@ -57,6 +57,9 @@ SIGNATURES: dict[str, tuple] = {
     "rebop_sg_cast_bf16": (_i, [_z, _v, _v, _v]),
     "rebop_sg_colsum": (_i, [_i, _i, _v, _i, _v, _v]),
     "rebop_sg_adam": (_i, [_z, _v, _v, _v, _v, _v, _f, _f, _f, _f, _f, _f, _v]),
+    "rebop_sg_mlp_train_forward": (_i, [_i, _v, _i, _i, _v, _v, _v, _v, _v, _v]),
+    "rebop_sg_mlp_backward_workspace": (c_size_t, [_i, _i, _v]),
+    "rebop_sg_mlp_backward": (_i, [_i, _i, _v, _v, _i, _v, _i, _v, _v, _v, _v, _v]),
     "rebop_sg_features": (_i, [_i, _v, _v, _v, _v, _d, _i, _v, _i, _v, _v]),
     "rebop_sg_head_offsets": (_i, [_i, _i, _i, _v, _i, _v, _v]),
     "rebop_sg_pack_kslices_bf16": (_i, [_i, _i, _v, _v, _v]),
@@ -178,6 +181,15 @@ def packed(W):
     Wp = torch.empty((W.shape[0] // 32, W.shape[1], 32), dtype=torch.bfloat16, device="cuda")
     pack_kslices(W, Wp)
     return Wp
+
+
+def _ints(values):
+    return (ctypes.c_int * len(values))(*values)
+
+
+def _ptrs(tensors):
+    """Host array of the tensors' device pointers."""
+    return (ctypes.c_void_p * len(tensors))(*[_p(t) for t in tensors])
 
 
 def _layer_table(Wp, bias):
@@ -316,45 +328,34 @@ class MLP:
         """X [B][IN] bf16 -> head [B][OUT] float32 (activations kept for backward)."""
         import torch
 
-        B = X.shape[0]
-        H = [X]
-        for l in range(self.depth):
-            # product, bias and activation in one launch (same values as
-            # gemm + bias_act)
-            if l < self.depth - 1:
-                h = torch.empty((B, self.dims[l + 1]), dtype=torch.bfloat16, device="cuda")
-                gemm_bias_act(H[-1], self.Wt[l], self.b[l], True, H=h, tb=True)
-                H.append(h)
-            else:
-                head = torch.empty((B, self.dims[l + 1]), dtype=torch.float32, device="cuda")
-                gemm_bias_act(H[-1], self.Wt[l], self.b[l], False, F=head, tb=True)
+        B, depth = X.shape[0], self.depth
+        H = [torch.empty((B, n), dtype=torch.bfloat16, device="cuda") for n in self.dims[1:-1]]
+        head = torch.empty((B, self.dims[-1]), dtype=torch.float32, device="cuda")
+        _ck(load().rebop_sg_mlp_train_forward(B, _p(X), X.shape[1], depth, _ints(self.dims), _ptrs(self.Wt),
+                                              _ptrs(self.b), _ptrs(H), _p(head), None))
         if keep:
-            self._H = H
+            self._H = [X] + H
         return head
 
     def backward(self, dhead):
-        """dhead [B][OUT] float32 -> (dW, db) per layer."""
+        """dhead [B][OUT] float32 -> (dW, db) per layer (views of one buffer)."""
         import torch
 
-        H = self._H
-        B = dhead.shape[0]
-        dW = [None] * self.depth
-        db = [None] * self.depth
-        dH = dhead.clone()
-        for l in reversed(range(self.depth)):
-            dZ = torch.empty((B, self.dims[l + 1]), dtype=torch.bfloat16, device="cuda")
-            if l == self.depth - 1:
-                cast_bf16(dH, dZ)
-            else:
-                relu_grad(dH, H[l + 1], dZ)
-            db[l] = torch.empty(self.dims[l + 1], dtype=torch.float32, device="cuda")
-            colsum(dH, db[l])
-            dW[l] = torch.empty((self.dims[l], self.dims[l + 1]), dtype=torch.float32, device="cuda")
-            gemm(H[l], dZ, dW[l], ta=True)
-            if l > 0:
-                dH = torch.empty((B, self.dims[l]), dtype=torch.float32, device="cuda")
-                gemm(dZ, self.Wb[l], dH, tb=True)
-        return dW, db
+        X, H = self._H[0], self._H[1:]
+        B, depth, lib = dhead.shape[0], self.depth, load()
+        dims = _ints(self.dims)
+        dhead = dhead.contiguous()
+        size = lib.rebop_sg_mlp_backward_workspace(B, depth, dims)
+        if size == 0:
+            raise _native.RebopError(3, "the batch and the widths must be multiples of 64")
+        work = torch.empty(size, dtype=torch.uint8, device="cuda")
+        shapes = list(zip(self.dims[:-1], self.dims[1:]))
+        weights = sum(m * n for m, n in shapes)
+        grads = torch.empty(weights + sum(self.dims[1:]), dtype=torch.float32, device="cuda")
+        _ck(lib.rebop_sg_mlp_backward(B, depth, dims, _p(dhead), dhead.shape[1], _p(X), X.shape[1], _ptrs(H),
+                                      _ptrs(self.Wb), _p(work), _p(grads), None))
+        parts = grads.split([m * n for m, n in shapes] + self.dims[1:])
+        return [g.view(s) for g, s in zip(parts, shapes)], list(parts[depth:])
 
     def step(self, dW, db, lr: float, b1=0.9, b2=0.999, eps=1e-8):
         self.t += 1

@@ -464,3 +464,72 @@ def test_nll_kernel_species_and_samples(sg, S, J, bounded):
     got = grad.double().cpu().numpy()
     assert np.allclose(got[:, :S * 3 * K], g[:, :S * 3 * K], rtol=1e-6, atol=1e-6 * np.abs(g).max())
     assert (got[:, S * 3 * K:] == 0).all()
+
+
+@pytest.mark.parametrize("B,width,depth", [(64, 64, 1), (64, 128, 2), (192, 192, 3), (448, 512, 5), (1088, 320, 4),
+                                           (128, 64, 10), (16384, 512, 3), (4096, 256, 5)])
+def test_training_passes_of_any_shape(sg, B, width, depth):
+    """Forward: the bits of the layer-by-layer products.  Backward: FP64
+    products of the same BF16 operands; a dZ on a rounding boundary may differ
+    by one BF16 step (2^-8 of itself), far below 2e-3 of the largest sum."""
+    import torch
+
+    mlp = sg.MLP(seed=B + depth, width=width, depth=depth)
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    X = torch.randn((B, sg.IN), generator=gen, device="cuda").to(torch.bfloat16)
+    dhead = torch.randn((B, sg.OUT), generator=gen, device="cuda")
+    head = mlp.forward(X)
+    H = list(mlp._H)
+    for l in range(depth):
+        ref = H[l].double() @ mlp.Wt[l].double().t() + mlp.b[l].double()
+        got = (head if l == depth - 1 else H[l + 1]).double()
+        if l < depth - 1:
+            ref = ref.clamp(min=0.0)
+        # FP32 accumulation of up to 512 terms, then (hidden) a BF16 rounding
+        tol = ref.abs().max() * (1e-5 + (0.0 if l == depth - 1 else 2.0 ** -8))
+        assert float((got - ref).abs().max()) <= float(tol), l
+    dW, db = mlp.backward(dhead)
+    dW2, db2 = mlp.backward(dhead)
+    for a, b in zip(dW + db, dW2 + db2):
+        assert torch.equal(a, b)  # a fixed order of summation
+    g = dhead.double()
+    for l in reversed(range(depth)):
+        dZ = g.float().to(torch.bfloat16).double()
+        rW, rb = H[l].double().t() @ dZ, g.sum(0)
+        assert dW[l].shape == rW.shape and db[l].shape == rb.shape
+        assert float((dW[l].double() - rW).abs().max()) <= 2e-3 * float(rW.abs().max()), l
+        assert float((db[l].double() - rb).abs().max()) <= 2e-3 * float(g.abs().sum(0).max()), l
+        g = (dZ @ mlp.Wb[l].double().t()) * (H[l].double() > 0)
+
+
+def test_training_passes_refuse_ragged_batches(sg):
+    import torch
+
+    from rebop_amd._native import RebopError
+
+    mlp = sg.MLP(seed=1, width=128, depth=2)
+    with pytest.raises(RebopError):
+        mlp.forward(torch.zeros((96, sg.IN), dtype=torch.bfloat16, device="cuda"))
+
+
+@pytest.mark.parametrize("Kd", [32, 96, 128, 224])
+def test_fused_epilogue_with_unaligned_outputs(sg, Kd):
+    """Outputs that start off a 16-byte boundary are written element by
+    element: the same values.  K off the 64-wide slices on the way."""
+    import torch
+
+    M, N = 64, 128
+    gen = torch.Generator(device="cuda").manual_seed(Kd)
+    A = torch.randn((M, Kd), generator=gen, device="cuda").to(torch.bfloat16)
+    Bt = torch.randn((N, Kd), generator=gen, device="cuda").to(torch.bfloat16)
+    bias = torch.randn(N, generator=gen, device="cuda")
+    H, F = torch.zeros((M, N), dtype=torch.bfloat16, device="cuda"), torch.zeros((M, N), device="cuda")
+    sg.gemm_bias_act(A, Bt, bias, True, H=H, F=F, tb=True)
+    Hu = torch.zeros(M * N + 8, dtype=torch.bfloat16, device="cuda")
+    Fu = torch.zeros(M * N + 8, device="cuda")
+    h, f = Hu[1:1 + M * N].view(M, N), Fu[3:3 + M * N].view(M, N)
+    sg.gemm_bias_act(A, Bt, bias, True, H=h, F=f, tb=True)
+    assert torch.equal(h.view(torch.int16), H.view(torch.int16)) and torch.equal(f, F)
+    assert (Hu[0] == 0) and (Hu[1 + M * N:] == 0).all() and (Fu[:3] == 0).all() and (Fu[3 + M * N:] == 0).all()
+    ref = (A.double() @ Bt.double().t() + bias.double()).clamp(min=0.0)
+    assert float((F.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
