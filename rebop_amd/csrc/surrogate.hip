@@ -329,13 +329,16 @@ __global__ void __launch_bounds__(256) gemm_nt_kernel(int M, int N, int K, const
 // The weight gradients of every layer in one launch: dW_l = H_l^T dZ_l, H_l
 // [B][m_l] and dZ_l [B][n_l] both with the contraction index b outermost.
 // A workgroup takes a 64 x 64 tile of one layer and a range of the batch
-// (split z of gridDim.y), 64 rows at a time: a thread reads 8 columns of 4
+// (split z), 64 rows at a time: a thread reads 8 columns of 4
 // rows, transposes them with byte permutes, and writes 4 consecutive b of
 // each column to LDS, from where the MFMA fragments are read.  The rows after
 // the current ones are on their way in registers meanwhile.  A layer at a
 // time would leave the chip a quarter full; all of them give 216 tiles (five
 // layers, width 512).  Splits write their sums to part[z], which
 // grad_reduce_kernel adds in order: no atomics, and the same bits every run.
+// Bound by LDS issue.  Five layers of width 512, batch 4096: 23.7 us (a launch
+// and a clear per layer with scattered LDS stores: 113 us; rows padded by four
+// elements instead of the chunk permutation: 29.5 us).
 constexpr int WG_MAXL = 8;
 struct WgradNet {
   const __bf16 *H[WG_MAXL], *dZ[WG_MAXL];
@@ -346,17 +349,24 @@ struct WgradNet {
   int layers;
 };
 
-__global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, float *__restrict__ part,
+__global__ void __launch_bounds__(256) wgrad_kernel(int units, int splits, WgradNet net, float *__restrict__ part,
                                                     size_t stride) {
-  constexpr int LD = 68; // 136 B rows: 8-byte accesses, at most two lanes per bank
+  // Rows of nine 16-byte chunks; chunk k of column c is stored at k ^ 2 (c / 16
+  // % 4), so that the 32 lanes of a store, four b of columns 8 apart, meet
+  // every bank once, as do 16 rows of a fragment.
+  constexpr int LD = 72;
   __shared__ __attribute__((aligned(16))) __bf16 T[2][2][64][LD]; // [buffer][H, dZ][column][b]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // the splits are a power of two and the fastest index, so consecutive
+  // workgroups, which go to different XCDs, share a tile and an XCD keeps to
+  // one range of the batch: a layer's operands over it fit its L2
+  const int tile = (int)blockIdx.x / splits, z = (int)blockIdx.x % splits;
   const __bf16 *H = net.H[0], *Z = net.dZ[0];
   int n = net.n[0], ldh = net.ldh[0], t0 = 0;
   size_t out = net.out[0];
 #pragma unroll
   for (int l = 1; l < WG_MAXL; ++l)
-    if (l < net.layers && (int)blockIdx.x >= net.tile0[l]) {
+    if (l < net.layers && tile >= net.tile0[l]) {
       H = net.H[l];
       Z = net.dZ[l];
       n = net.n[l];
@@ -364,9 +374,9 @@ __global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, flo
       t0 = net.tile0[l];
       out = net.out[l];
     }
-  const int t = (int)blockIdx.x - t0, tn = n / 64, m0 = t / tn * 64, n0 = t % tn * 64;
-  const int ubeg = (int)((int64_t)units * blockIdx.y / gridDim.y);
-  const int uend = (int)((int64_t)units * (blockIdx.y + 1) / gridDim.y);
+  const int t = tile - t0, tn = n / 64, m0 = t / tn * 64, n0 = t % tn * 64;
+  const int ubeg = (int)((int64_t)units * z / splits);
+  const int uend = (int)((int64_t)units * (z + 1) / splits);
   const int side = tid >> 7, cg = tid & 7, kq = (tid & 127) >> 3;
   const size_t ld = side ? (size_t)n : (size_t)ldh;
   const __bf16 *src = (side ? Z + n0 : H + m0) + (size_t)(4 * kq) * ld + 8 * cg;
@@ -382,6 +392,7 @@ __global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, flo
     }
   };
   auto lstore = [&](int buf) {
+    const int at = 4 * kq ^ 16 * (cg >> 1);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       uint2 lo, hi; // columns 2 w and 2 w + 1, rows 0..3
@@ -389,17 +400,12 @@ __global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, flo
       lo.y = __builtin_amdgcn_perm(r[3][w], r[2][w], 0x05040100u);
       hi.x = __builtin_amdgcn_perm(r[1][w], r[0][w], 0x07060302u);
       hi.y = __builtin_amdgcn_perm(r[3][w], r[2][w], 0x07060302u);
-      *(uint2 *)&T[buf][side][8 * cg + 2 * w][4 * kq] = lo;
-      *(uint2 *)&T[buf][side][8 * cg + 2 * w + 1][4 * kq] = hi;
+      *(uint2 *)&T[buf][side][8 * cg + 2 * w][at] = lo;
+      *(uint2 *)&T[buf][side][8 * cg + 2 * w + 1][at] = hi;
     }
   };
   auto frag = [&](int buf, int s, int c, int k) { // 8 consecutive b of column c
-    bf16x8 v;
-    uint2 a[2];
-    a[0] = *(const uint2 *)&T[buf][s][c][k];
-    a[1] = *(const uint2 *)&T[buf][s][c][k + 4];
-    __builtin_memcpy(&v, a, sizeof v);
-    return v;
+    return *(const bf16x8 *)&T[buf][s][c][k ^ 16 * (c >> 4 & 3)];
   };
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   floatx4 acc[2][2];
@@ -430,7 +436,7 @@ __global__ void __launch_bounds__(256) wgrad_kernel(int units, WgradNet net, flo
     __syncthreads();
     buf ^= 1;
   }
-  float *o = part + stride * blockIdx.y + out;
+  float *o = part + stride * z + out;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -654,36 +660,43 @@ __device__ __forceinline__ double item_feature(const ItemInputs &v, const double
   }
 }
 
-__device__ __forceinline__ void item_features(uint32_t p, uint32_t i, const double *__restrict__ rates,
-                                              const int64_t *__restrict__ x0, double tmax, int nb_steps,
-                                              float (&f)[REBOP_SG_FEATURES], float &e0f, float &s0f) {
-  const ItemInputs v = item_inputs(p, i, rates, x0, tmax, nb_steps);
-  double lg[7];
-#pragma unroll
-  for (int j = 0; j < 7; ++j) lg[j] = item_log(v, j);
-#pragma unroll
-  for (int j = 0; j < REBOP_SG_FEATURES; ++j) f[j] = (float)item_feature(v, lg, tmax, j);
-  e0f = (float)v.e0;
-  s0f = (float)v.s0;
-}
-
 // X[b][0..ldx) = item b's features, then zeros; bound[b][s] (nullable) = the
 // count that bounds species s (E = E0 - ES, S <= S0, ES <= E0, P <= S0).
-__global__ void features_kernel(int B, const uint32_t *__restrict__ item_point,
-                                const uint32_t *__restrict__ item_sample, const double *__restrict__ rates,
-                                const int64_t *__restrict__ x0, double tmax, int nb_steps,
-                                __bf16 *__restrict__ X, int ldx, float *__restrict__ bound) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// Four threads per item: thread q computes logs 2q and 2q + 1 (of seven),
+// which the four share through LDS, and features 4q .. 4q+3.  A thread per
+// item took seven logarithms in a row on 16 workgroups and wrote its row two
+// bytes at a time (4096 items: 13.1 us, now 4.8 us).  wide: rows of X may be written eight bytes at a time.
+__global__ void __launch_bounds__(256) features_kernel(int B, const uint32_t *__restrict__ item_point,
+                                                       const uint32_t *__restrict__ item_sample,
+                                                       const double *__restrict__ rates,
+                                                       const int64_t *__restrict__ x0, double tmax, int nb_steps,
+                                                       __bf16 *__restrict__ X, int ldx, float *__restrict__ bound,
+                                                       bool wide) {
+  static_assert(REBOP_SG_FEATURES == 16, "four threads x four features per item");
+  __shared__ double lg[64][9]; // rows 72 B apart
+  const int row = threadIdx.x >> 2, q = threadIdx.x & 3;
+  const int b = blockIdx.x * 64 + row;
+  ItemInputs v{1.0, 1.0, 1.0, 1.0, 1.0, 1.0};
+  if (b < B) v = item_inputs(item_point[b], item_sample[b], rates, x0, tmax, nb_steps);
+  lg[row][2 * q] = item_log(v, 2 * q);
+  if (q < 3) lg[row][2 * q + 1] = item_log(v, 2 * q + 1);
+  __syncthreads();
   if (b >= B) return;
-  float f[REBOP_SG_FEATURES], e0, s0;
-  item_features(item_point[b], item_sample[b], rates, x0, tmax, nb_steps, f, e0, s0);
-  for (int c = 0; c < ldx; ++c) X[(size_t)b * ldx + c] = (__bf16)(c < REBOP_SG_FEATURES ? f[c] : 0.f);
-  if (bound) {
-    bound[4 * b + 0] = e0;
-    bound[4 * b + 1] = s0;
-    bound[4 * b + 2] = e0;
-    bound[4 * b + 3] = s0;
+  __bf16 h[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) h[j] = (__bf16)(float)item_feature(v, lg[row], tmax, 4 * q + j);
+  __bf16 *x = X + (size_t)b * ldx;
+  if (wide) {
+    const __bf16 z[4] = {};
+    __builtin_memcpy(__builtin_assume_aligned(x + 4 * q, 8), h, sizeof h);
+    for (int c = REBOP_SG_FEATURES + 4 * q; c < ldx; c += 16)
+      __builtin_memcpy(__builtin_assume_aligned(x + c, 8), z, sizeof z);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[4 * q + j] = h[j];
+    for (int c = REBOP_SG_FEATURES + q; c < ldx; c += 4) x[c] = (__bf16)0.f;
   }
+  if (bound) bound[4 * (size_t)b + q] = (float)(q & 1 ? v.s0 : v.e0);
 }
 
 // head[b][s*3K + K + c] += ln bound[b][s] for the negative-binomial
@@ -713,7 +726,7 @@ __global__ void head_offsets_kernel(int B, int S, int K, float *__restrict__ hea
 // 16x16x32 MFMAs over k slices 0, 32, 64, ... (a product of two BF16 values
 // is exact in FP32, so which operand is A does not matter), then + bias,
 // ReLU and the BF16 cast -- the bits of the layer-by-layer forward pass.
-// FEAT: the input layer is item_features of items m0.. (columns >=
+// FEAT: the input layer is item_feature of items m0.. (columns >=
 // REBOP_SG_FEATURES zero) and the last layer adds head_offsets_kernel's
 // ln bound terms, so one launch turns (point, sample) items into mixture
 // parameters; otherwise X [M][ldx] is the input.
@@ -939,7 +952,7 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(int M, const __bf16 *__r
   if (FEAT) {
     // four threads per item: thread q computes logs 2q, 2q+1 (of seven),
     // which the item's threads share through LDS, then features 4q .. 4q+3
-    // (the arithmetic of item_features, so the bits of features_kernel)
+    // (the arithmetic of item_feature, so the bits of features_kernel)
     static_assert(REBOP_SG_FEATURES == 16 && MLP_BM * 4 == 512, "four threads x four features per item");
     const int item = tid >> 2, q = tid & 3;
     ItemInputs v{1.0, 1.0, 1.0, 1.0, 1.0, 1.0};
@@ -1410,10 +1423,8 @@ bool train_plan(int B, int depth, const int *dims, TrainPlan &p) {
     p.nbias += dims[l];
   }
   p.units = B / 64;
-  // about 1024 workgroups (four to a CU) of at least 128 rows each
-  size_t z = 1024 / tiles;
-  if (z > (size_t)p.units / 2) z = (size_t)p.units / 2;
-  p.splits = z < 1 ? 1 : z > 32 ? 32 : (int)z;
+  // a power of two: about 1024 workgroups (four to a CU) of at least 128 rows each
+  while (p.splits < 32 && 2 * p.splits <= p.units / 2 && 2 * p.splits * tiles <= 1024) p.splits *= 2;
   p.dz = (size_t)B * p.nbias;
   p.colsum = (size_t)p.units * p.nbias;
   p.part = p.splits > 1 ? p.weights * (size_t)p.splits : 0;
@@ -1549,7 +1560,8 @@ int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead,
       tiles += (dims[l] / 64) * (dims[l + 1] / 64);
       at += (size_t)dims[l] * dims[l + 1];
     }
-    hipLaunchKernelGGL(sg::wgrad_kernel, dim3(tiles, p.splits), dim3(256), 0, s, p.units, net, wout, p.weights);
+    hipLaunchKernelGGL(sg::wgrad_kernel, dim3(tiles * p.splits), dim3(256), 0, s, p.units, p.splits, net, wout,
+                       p.weights);
   }
   const unsigned blocks = (p.splits > 1 ? (unsigned)(p.weights / 1024) : 0u) + nblk((size_t)p.nbias, 64);
   hipLaunchKernelGGL(sg::grad_reduce_kernel, dim3(blocks), dim3(256), 0, s, p.splits, p.weights, p.weights, part,
@@ -1603,9 +1615,9 @@ int rebop_sg_features(int B, const uint32_t *item_point, const uint32_t *item_sa
                       const double *rates, const int64_t *x0, double tmax, int nb_steps, void *X,
                       int ldx, float *bound, void *stream) {
   if (ldx < REBOP_SG_FEATURES) return 3;
-  hipLaunchKernelGGL(sg::features_kernel, dim3(nblk((size_t)B, 256)), dim3(256), 0,
-                     (hipStream_t)stream, B, item_point, item_sample, rates, x0, tmax, nb_steps,
-                     (__bf16 *)X, ldx, bound);
+  const bool wide = (uintptr_t)X % 8 == 0 && ldx % 4 == 0;
+  hipLaunchKernelGGL(sg::features_kernel, dim3(nblk((size_t)B, 64)), dim3(256), 0, (hipStream_t)stream, B,
+                     item_point, item_sample, rates, x0, tmax, nb_steps, (__bf16 *)X, ldx, bound, wide);
   return ret(hipGetLastError());
 }
 

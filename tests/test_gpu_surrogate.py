@@ -533,3 +533,29 @@ def test_fused_epilogue_with_unaligned_outputs(sg, Kd):
     assert (Hu[0] == 0) and (Hu[1 + M * N:] == 0).all() and (Fu[:3] == 0).all() and (Fu[3 + M * N:] == 0).all()
     ref = (A.double() @ Bt.double().t() + bias.double()).clamp(min=0.0)
     assert float((F.double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("B,ldx,off", [(1, 64, 0), (63, 16, 0), (65, 20, 0), (130, 67, 0), (100, 64, 1)])
+def test_features_of_any_count_and_row(sg, B, ldx, off):
+    """Ragged item counts, rows off the eight-byte stores and past the
+    features: the values of the FP64 reference's BF16 rounding (a device log10
+    may differ in its last bit, one BF16 step at most)."""
+    import torch
+
+    from oracle import surrogate_ref as ref
+
+    rates, x0 = sg.sample_points(50, seed=B)
+    rng = np.random.default_rng(B)
+    ip, isamp = rng.integers(0, 50, B).astype(np.int32), rng.integers(1, sg.NB + 1, B).astype(np.int32)
+    dev = lambda a: torch.as_tensor(a, device="cuda")  # noqa: E731
+    buf = torch.full((B * ldx + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+    X = buf[off:off + B * ldx].view(B, ldx)
+    bound = torch.full((B + 1, 4), -1.0, device="cuda")
+    sg.features(dev(ip), dev(isamp), dev(rates), dev(x0), X, bound[:B])
+    Xr, br = ref.features(rates[ip], x0[ip], isamp.astype(np.float64), sg.TMAX, sg.NB, 64, with_offsets=True)
+    got = X.double().cpu().numpy()
+    want = np.zeros((B, ldx))
+    want[:, :16] = ref.bf16(Xr)[:, :16]
+    assert (np.abs(got - want) <= np.abs(want) * 2.0**-7 + 1e-30).all()
+    assert np.array_equal(bound[:B].double().cpu().numpy(), br) and (bound[B] == -1).all()
+    assert (buf[:off] == 7).all() and (buf[off + B * ldx:] == 7).all()
