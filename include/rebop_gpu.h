@@ -77,7 +77,8 @@ enum rebop_kernel_kind {
   REBOP_KERNEL_SPECIALIZED = 16,
   /* flags: 2 or 4 lanes per trajectory, sharing the Philox blocks and ln of
    * the next draws (PLAIN | SPECIALIZED grid runs; AUTO picks them when the
-   * run has too few trajectories for more than one wave per SIMD) */
+   * run has too few trajectories for more than one wave per SIMD, and takes
+   * 16 lanes, reported as GROUP4, for the fewest) */
   REBOP_KERNEL_GROUP2 = 32,
   REBOP_KERNEL_GROUP4 = 64,
   /* flag: a persistent specialised grid or target run finishes every

@@ -121,6 +121,9 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "  __device__ __forceinline__ void store_state(const X &x, double *st, uint64_t stride) const { rebop::reg_store_state(x, st, stride, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ void write_counts(const X &x, int64_t *dst, uint64_t stride) const { rebop::reg_write_counts(x, dst, stride, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ void write_raw(const X &x, int64_t *dst, uint64_t stride) const { rebop::reg_write_raw(x, dst, stride, " + Ss + "); }\n";
+  s += "  __device__ __forceinline__ void write_raw_buffer(const X &x, rebop::WordBuffer b, uint32_t at, uint32_t stride) const { rebop::reg_write_raw_buffer(x, b, at, stride, " + Ss + "); }\n";
+  s += "  __device__ __forceinline__ bool small(const X &x) const { return rebop::reg_small(x, " + Ss + "); }\n";
+  s += "  __device__ __forceinline__ void write_small(const X &x, int64_t *dst) const { rebop::reg_write_small(x, dst, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ bool in_range(const X &x) const { return rebop::reg_in_range(x, " + Ss + "); }\n";
   // make_cumrates over Rate::rate
   s += "  __device__ __forceinline__ double props(X &x, C &cum) const {\n";
@@ -250,16 +253,23 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "  if (threadIdx.x < 4) blk_ctr[threadIdx.x] = 0ull;\n";
   s += "  for (uint32_t w = threadIdx.x; w < 512u; w += blockDim.x)\n";
   s += "    (&ln_lds[0][0])[w] = (&rebop_ln_table[0][0])[w];\n";
-  s += "  const bool lds_grid = run.mode == REBOP_MODE_GRID && run.grid && run.nb_steps < REBOP_GRID_LDS;\n";
+  s += "  const uint64_t samples = rebop::run_samples(run);\n";
+  s += "  const bool lds_grid = run.mode != REBOP_MODE_EVENTS && run.grid && samples <= REBOP_GRID_LDS;\n";
   s += "  if (lds_grid)\n";
-  s += "    for (uint32_t w = threadIdx.x; w <= (uint32_t)run.nb_steps; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
+  s += "    for (uint32_t w = threadIdx.x; w < samples; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
+  s += "  if (lds_grid && threadIdx.x < REBOP_GRID_PAD) grid_lds[samples + threadIdx.x] = __builtin_nan(\"\");\n";
   s += "  __syncthreads();\n";
+  s += "  const bool straight = rebop::group_straight(run, " + Ss + ");\n";
   s += "  JitNet<false> net;\n";
   s += "  const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
-  s += "  const rebop::LaneTotals acc =\n";
-  s += "      run.mode == REBOP_MODE_EVENTS ? rebop::lane_events_group<JitNet<false>, K>(net, run, gtid, ln_lds)\n";
-  s += "      : lds_grid ? rebop::lane_loop_group<JitNet<false>, K, true>(net, run, gtid, ln_lds, grid_lds)\n";
-  s += "                 : rebop::lane_loop_group<JitNet<false>, K, false>(net, run, gtid, ln_lds, nullptr);\n";
+  s += "  rebop::LaneTotals acc;\n";
+  // (a launch with 16 lanes is always one of straight rounds)
+  s += "  if constexpr (K == 16) acc = rebop::lane_loop_group<JitNet<false>, K, true, true>(net, run, gtid, ln_lds, grid_lds);\n";
+  s += "  else acc = run.mode == REBOP_MODE_EVENTS\n";
+  s += "          ? (run.rec_offsets ? rebop::lane_events_group<JitNet<false>, K, true>(net, run, gtid, ln_lds)\n";
+  s += "                             : rebop::lane_events_group<JitNet<false>, K, false>(net, run, gtid, ln_lds))\n";
+  s += "      : lds_grid && straight ? rebop::lane_loop_group<JitNet<false>, K, true, true>(net, run, gtid, ln_lds, grid_lds)\n";
+  s += "                             : rebop::lane_loop_group<JitNet<false>, K, false, false>(net, run, gtid, ln_lds, nullptr);\n";
   s += "  rebop::flush_totals(acc, run, blk_ctr);\n";
   s += "}\n";
   // REBOP_JIT_WAVES_PER_EU=<n>: ask the compiler to fit n waves per SIMD in
@@ -274,6 +284,8 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_sweep(rebop_dev_run run) { jit_body<true>(run); }\n";
   s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g2(rebop_dev_run run) { jit_body_group<2>(run); }\n";
   s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g4(rebop_dev_run run) { jit_body_group<4>(run); }\n";
+  if (!cap) // with a draw cap every round is stepped through, and long ones only cost code
+    s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g16(rebop_dev_run run) { jit_body_group<16>(run); }\n";
   return s;
 }
 
@@ -438,6 +450,8 @@ int jit_get(const std::string &src, JitKernel *out, std::string *err) {
   if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_sweep, k.mod, "rebop_ssa_jit_sweep");
   if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_g2, k.mod, "rebop_ssa_jit_g2");
   if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_g4, k.mod, "rebop_ssa_jit_g4");
+  if (he == hipSuccess && src.find("rebop_ssa_jit_g16") != std::string::npos)
+    he = hipModuleGetFunction(&k.fn_g16, k.mod, "rebop_ssa_jit_g16");
   if (he != hipSuccess) {
     *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(he);
     return -1;
@@ -475,8 +489,9 @@ int jit_compile_only(const std::string &src, size_t *code_size, std::string *err
 size_t jit_dynamic_lds(const rebop_dev_run &run) {
   // the LDS copy of the sample times (jit_body, jit_body_group; a grid run
   // always has its table)
-  const bool grid_lds = !run.rates && run.mode == REBOP_MODE_GRID && run.nb_steps < REBOP_GRID_LDS;
-  return grid_lds ? sizeof(double) * (size_t)(run.nb_steps + 1u) : 0u;
+  if (run.rates || run.mode == REBOP_MODE_EVENTS) return 0u;
+  const uint64_t samples = run_samples(run);
+  return samples <= REBOP_GRID_LDS ? sizeof(double) * (size_t)(samples + REBOP_GRID_PAD) : 0u;
 }
 
 hipError_t jit_occupancy(const JitKernel &k, int threads, size_t lds, int *blocks_per_cu) {
@@ -487,7 +502,7 @@ hipError_t jit_launch(const JitKernel &k, const rebop_dev_run &run, int blocks, 
                       hipStream_t stream, int group) {
   rebop_dev_run arg = run;
   void *params[] = {&arg};
-  hipFunction_t f = run.rates ? k.fn_sweep : group == 4 ? k.fn_g4 : group == 2 ? k.fn_g2 : k.fn;
+  hipFunction_t f = run.rates ? k.fn_sweep : group == 16 ? k.fn_g16 : group == 4 ? k.fn_g4 : group == 2 ? k.fn_g2 : k.fn;
   return hipModuleLaunchKernel(f, (unsigned)blocks, 1, 1, (unsigned)threads, 1, 1,
                                (unsigned)jit_dynamic_lds(run), stream, params, nullptr);
 }

@@ -32,6 +32,7 @@ struct JitKernel {
   hipFunction_t fn_sweep = nullptr;
   hipFunction_t fn_g2 = nullptr; // 2 lanes per trajectory (plain launches)
   hipFunction_t fn_g4 = nullptr; // 4 lanes per trajectory
+  hipFunction_t fn_g16 = nullptr; // 16 lanes per trajectory (not with a draw cap)
 };
 
 // Kernel source for a network of S species and the given reactions; with
@@ -46,8 +47,8 @@ int jit_compile_only(const std::string &src, size_t *code_size, std::string *err
 // Dynamic LDS bytes a launch of `run` takes (the LDS copy of the sample times).
 size_t jit_dynamic_lds(const rebop_dev_run &run);
 hipError_t jit_occupancy(const JitKernel &k, int threads, size_t lds, int *blocks_per_cu);
-// group = lanes per trajectory (1, 2 or 4; 2 and 4 only for plain, non-sweep
-// grid/target runs)
+// group = lanes per trajectory (1, 2, 4 or 16; above 1 only for plain, non-sweep
+// runs, 16 only without a draw cap)
 hipError_t jit_launch(const JitKernel &k, const rebop_dev_run &run, int blocks, int threads,
                       hipStream_t stream, int group = 1);
 

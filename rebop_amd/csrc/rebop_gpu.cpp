@@ -1103,6 +1103,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   // a large network's kernel is free (AUTO), not asked for as REBOP_KERNEL_LDS
   bool any_lds = kernel == REBOP_KERNEL_AUTO || kernel == kKernelAnyLds;
   if (kernel == kKernelAnyLds) kernel = REBOP_KERNEL_LDS;
+  const bool any_group = kernel == REBOP_KERNEL_AUTO; // the lanes per trajectory are free
   if (kernel == REBOP_KERNEL_AUTO && g->tune_kernel >= 0 && threads == 0) {
     kernel = g->tune_kernel;
     threads = g->tune_threads;
@@ -1231,6 +1232,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   // lanes per trajectory: asked for, or (AUTO) when even 4 (2) lanes per
   // trajectory leave at most one wave per SIMD
   int group = (kernel & REBOP_KERNEL_GROUP4) ? 4 : (kernel & REBOP_KERNEL_GROUP2) ? 2 : 1;
+  const uint64_t lanes = (uint64_t)g_dev.cus * 4u * 64u; // one wave per SIMD
   if (group > 1) {
     if (!spec)
       return fail(REBOP_ERR_UNSUPPORTED,
@@ -1239,12 +1241,19 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
       return fail(REBOP_ERR_UNSUPPORTED,
                   "lanes per trajectory > 1 applies to plain runs without rate tables");
   } else if (variant == REBOP_KERNEL_AUTO && spec && !run.rates) {
-    const uint64_t lanes = (uint64_t)g_dev.cus * 4u * 64u;
     if (run.n_traj * 4u <= lanes)
       group = 4;
     else if (run.n_traj * 2u <= lanes)
       group = 2;
   }
+  // Sixteen lanes where they too leave one wave per SIMD, unless four were
+  // asked for: a draw (a Philox block and a logarithm, a third of an event's
+  // instructions with four lanes) then costs a sixteenth of its own.  4096 SIR
+  // trajectories advanced to two times, a call: 772 us with four lanes and
+  // every test, 570 us with sixteen in straight rounds (692 us when those
+  // end every four draws).
+  if (group == 4 && any_group && spec && !run.draw_cap && run.n_traj * 16u <= lanes && rebop::group_straight(run, S))
+    group = 16;
   const bool persistent = group == 1 && variant != REBOP_KERNEL_PLAIN;
   const int shape = spec ? -1 : pick_reg_shape(S, R);
   if (!spec && shape < 0)
@@ -1273,7 +1282,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   if (blocks > 0x7fffffffull) return fail(REBOP_ERR_VALUE, "too many trajectories for one launch");
   const int kind = (persistent ? REBOP_KERNEL_PERSISTENT : REBOP_KERNEL_PLAIN) |
                    (spec ? REBOP_KERNEL_SPECIALIZED : 0) |
-                   (group == 4 ? REBOP_KERNEL_GROUP4 : group == 2 ? REBOP_KERNEL_GROUP2 : 0);
+                   (group >= 4 ? REBOP_KERNEL_GROUP4 : group == 2 ? REBOP_KERNEL_GROUP2 : 0);
   // tail hand-off (see rebop_dev_run): a wave spills at most spill_below
   // trajectories, once, so the arrays need (waves x spill_below) entries
   const uint32_t below = tail_lanes();

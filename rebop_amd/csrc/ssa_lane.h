@@ -128,6 +128,54 @@ __device__ __forceinline__ void reg_write_raw(const double (&x)[MS], int64_t *ds
     if (s < (int)S) dst[(uint64_t)s * stride] = (int64_t)rebop_f64_bits(x[s]);
 }
 
+// A buffer of `n` 8-byte words at p (below 2^31 of them): stores at a word's
+// index, dropped where it is past the end.
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef __amdgpu_buffer_rsrc_t WordBuffer;
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+__device__ void word_buffer_store(u32x2_t v, WordBuffer buf, int index, int offset, int soffset,
+                                  int aux) __asm("llvm.amdgcn.struct.ptr.buffer.store.v2i32");
+__device__ __forceinline__ WordBuffer word_buffer(void *p, uint32_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 8, (int)n, 0x00020000);
+}
+#else
+struct WordBuffer {};
+__device__ __forceinline__ WordBuffer word_buffer(void *, uint32_t) { return WordBuffer{}; }
+#endif
+// reg_write_raw to word `at`, the species `stride` words apart
+template <int MS>
+__device__ __forceinline__ void reg_write_raw_buffer(const double (&x)[MS], WordBuffer buf, uint32_t at,
+                                                     uint32_t stride, uint32_t S) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+  for (int s = 0; s < MS; ++s)
+    if (s < (int)S) {
+      const uint64_t b = rebop_f64_bits(x[s]);
+      word_buffer_store(u32x2_t{(uint32_t)b, (uint32_t)(b >> 32)}, buf, (int)at, 0, (int)(s * stride * 8u), 0);
+    }
+#endif
+}
+
+// Counts in [0, 2^50), tested like reg_in_range, and their conversion: adding
+// 1.5 2^52 leaves the integer (also a slightly negative one) in the low bits.
+template <int MS>
+__device__ __forceinline__ bool reg_small(const double (&x)[MS], uint32_t S) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int s = 0; s < MS; ++s)
+    if (s < (int)S) {
+      const uint32_t h = (uint32_t)(rebop_f64_bits(x[s]) >> 32);
+      m = m > h ? m : h;
+    }
+  return m < 0x43100000u;
+}
+template <int MS>
+__device__ __forceinline__ void reg_write_small(const double (&x)[MS], int64_t *dst, uint32_t S) {
+#pragma unroll
+  for (int s = 0; s < MS; ++s)
+    if (s < (int)S) dst[s] = (int64_t)(rebop_f64_bits(x[s] + 0x1.8p52) - 0x4338000000000000ull);
+}
+
 template <int MS>
 __device__ __forceinline__ bool reg_in_range(const double (&x)[MS], uint32_t S) {
   // the largest high word, as unsigned, is below 2^52's unless a count is
@@ -193,13 +241,19 @@ __device__ __forceinline__ double hit_cap(const rebop_dev_run &run, LaneTotals &
   return 0.0;
 }
 
+// How far above the usual totals' lower end `tot` is: kUsualSpan or more if it
+// is not a usual total.
+constexpr uint32_t kUsualSpan = 1400u << 20;
+__device__ __forceinline__ uint32_t usual_distance(double tot) {
+  return (uint32_t)(rebop_f64_bits(tot) >> 32) - ((1023u - 700u) << 20);
+}
+
 // Whether a total propensity lies in [2^-700, 2^700): positive, finite, and
 // far from where a division of an exponential (0 or 2^-53 .. 37) by it needs
 // scaling.  One range test of the high word stands for the tests for zero,
 // negative, NaN and infinite totals, which then cost nothing per event.
 __device__ __forceinline__ bool usual_total(double tot) {
-  const uint32_t hi = (uint32_t)(rebop_f64_bits(tot) >> 32);
-  return hi - ((1023u - 700u) << 20) < (1400u << 20);
+  return usual_distance(tot) < kUsualSpan;
 }
 
 // E / tot, correctly rounded, for a usual total: the reciprocal refined by two
@@ -414,13 +468,15 @@ __device__ __forceinline__ LaneTotals lane_loop(Net &net, const rebop_dev_run &r
   return acc;
 }
 
-// Lane q of each aligned group of K lanes (K = 2 or 4) reads `v` from lane Q
-// of its group: one DPP quad permutation per 32-bit half, no LDS traffic.
+// Lane q of each aligned group of K lanes (K = 2, 4 or 16) reads `v` from
+// lane Q of its group: one DPP move per 32-bit half (a quad permutation, or a
+// broadcast within a row of 16), no LDS traffic.
 template <int K, int Q>
 __device__ __forceinline__ double group_read(double v) {
-  static_assert(K == 2 || K == 4, "groups of 2 or 4 lanes");
-  constexpr int ctrl = K == 4 ? (Q | (Q << 2) | (Q << 4) | (Q << 6))
-                              : (Q | (Q << 2) | ((2 + Q) << 4) | ((2 + Q) << 6));
+  static_assert(K == 2 || K == 4 || K == 16, "groups of 2, 4 or 16 lanes");
+  constexpr int ctrl = K == 16  ? 0x150 + Q
+                       : K == 4 ? (Q | (Q << 2) | (Q << 4) | (Q << 6))
+                                : (Q | (Q << 2) | ((2 + Q) << 4) | ((2 + Q) << 6));
   const uint64_t b = rebop_f64_bits(v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, ctrl, 0xF, 0xF, false);
   const uint32_t hi =
@@ -428,13 +484,36 @@ __device__ __forceinline__ double group_read(double v) {
   return rebop_f64_from_bits(((uint64_t)hi << 32) | lo);
 }
 
+// The same for a q that is a constant once the caller's loop is unrolled, or
+// (groups of 16, whose careful rounds are not) known at run time.
 template <int K>
 __device__ __forceinline__ double group_read(double v, int q) {
-  switch (q) {
-  case 0: return group_read<K, 0>(v);
-  case 1: return group_read<K, 1>(v);
-  case 2: if constexpr (K == 4) return group_read<K, 2>(v); else return v;
-  default: if constexpr (K == 4) return group_read<K, 3>(v); else return v;
+  if constexpr (K == 16) {
+    const int at = (int)((__lane_id() & ~15u) + (uint32_t)q) * 4;
+    const uint64_t b = rebop_f64_bits(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)(uint32_t)b);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute(at, (int)(uint32_t)(b >> 32));
+    return rebop_f64_from_bits(((uint64_t)hi << 32) | lo);
+  } else {
+    switch (q) {
+    case 0: return group_read<K, 0>(v);
+    case 1: return group_read<K, 1>(v);
+    case 2: if constexpr (K == 4) return group_read<K, 2>(v); else return v;
+    default: if constexpr (K == 4) return group_read<K, 3>(v); else return v;
+    }
+  }
+}
+
+// f(GroupStep<q>{}) for q = 0 .. K - 1
+template <int Q>
+struct GroupStep {
+  static constexpr int q = Q;
+};
+template <int K, int Q = 0, class F>
+__device__ __forceinline__ void group_steps(F &&f) {
+  if constexpr (Q < K) {
+    f(GroupStep<Q>{});
+    group_steps<K, Q + 1>(f);
   }
 }
 
@@ -442,7 +521,7 @@ __device__ __forceinline__ double group_read(double v, int q) {
 // every SIMD more than one wave (there the time is one trajectory's serial
 // event chain, and the Philox block + ln of each draw is most of an event).
 // Lane `sub` of a group computes the block of draw (draw + sub) of the group's
-// trajectory; the group then runs up to K iterations of the state machine,
+// trajectory; the group then runs K iterations of the state machine,
 // iteration q using block q (read from lane q by DPP).  That is exactly the
 // draw each iteration would take: every event or overshoot consumes the next
 // draw, and a trajectory in an absorbing state never draws again (its counts
@@ -452,20 +531,42 @@ __device__ __forceinline__ double group_read(double v, int q) {
 // run.resume the trajectory of spill entry j (the tail of a persistent
 // launch, continued from its written-out state).
 //
-// One wave per SIMD issues every instruction of the chain itself, so the
-// loop keeps memory latency off that chain: `ln_tab` is the workgroup's LDS
-// copy of the ln table, whose rows for the next round's draws are read while
-// this round's events run (the next round's blocks are (draw + K + sub),
-// since a round either consumes K draws or ends the drawing for good), and
-// `grid_lds` its LDS copy of the sample times, read at every iteration while
-// the division runs.  No vector-memory wait is left in the loop, so the
-// sample stores are never waited for.  GridLds: grid_lds holds the sample
-// times (else the next one is carried, computed at each sample, for grids too
-// long for LDS).
-template <class Net, int K, bool GridLds>
+// A wave alone on its SIMD issues an instruction every five cycles or so, and
+// a branch costs it 30 to 60 cycles (compare, mask, skip, restore).  In nine
+// iterations of ten some of its sixteen trajectories records a sample while
+// the others fire, so both paths were issued and branched over.  Now an
+// iteration has one path: a trajectory that records takes no jump (reaction
+// MR is none) and keeps its total.  An absorbing state has total 0, whose
+// quotient is NaN, which is not at or below any sample time: it records
+// without a test of its own.  Draws and overshoots are not counted along the
+// way: until it is absorbed, a trajectory takes a draw in every iteration and
+// overshoots once per sample.  The range of the counts is checked once a round.
+//
+// Straight rounds (sample times in LDS, an output below 2^31 counts or none, no
+// draw cap) have no branch at all.  Samples are stored with buffer instructions whose
+// bounds check drops the lanes that have none.  A trajectory past its last
+// sample time reads NaN for the next, so it keeps recording, out of bounds,
+// until the round's end.  Totals that are not usual ones (an absorbed
+// trajectory's above all) are noticed at the end of the round, which is then
+// done again with the tests (the stores are the same).  10^4 SIR
+// trajectories of 250 samples, a call: 636 us with both paths branched over,
+// 557 us with one path and the tests, 488 us in straight rounds (59 vector
+// instructions an iteration with four lanes, 51 with sixteen).
+//
+// Memory latency stays off the chain: `ln_tab` is the workgroup's LDS copy of
+// the ln table, whose rows for the next round's draws are read while this
+// round's events run (the next round's blocks are (draw + K + sub), since a
+// round either consumes K draws or ends the drawing for good), and
+// `grid_lds` its LDS copy of the sample times, followed by REBOP_GRID_PAD
+// NaNs, read an iteration ahead.  No vector-memory wait is left
+// in the loop, so the sample stores are never waited for.  GridLds: grid_lds
+// holds the sample times (else the next one is carried, computed at each
+// sample, for grids too long for LDS).
+template <class Net, int K, bool GridLds, bool Straight>
 __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_run &run,
                                                       uint64_t gtid, const double (*ln_tab)[4],
                                                       const double *grid_lds) {
+  constexpr bool FAST = GridLds && Straight && !Net::kCap;
   LaneTotals acc;
   const uint64_t n = run.n_traj;
   const uint64_t e = gtid / K; // group index
@@ -491,45 +592,80 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
   for (int r = 0; r < Net::MR; ++r) cum[r] = 0.0;
   net.start(run, jl);
   double t;
-  uint64_t draw, mark;
-  uint32_t i = 0, ov = 0;
-  bool capped = false;
+  uint64_t draw;
+  uint32_t i = 0;
+  bool dead = false; // absorbing, stopped by the cap, or finished: tot is 0
   if (run.resume) {
     net.load_state(x, run.spill_x + e, run.spill_cap);
     t = run.spill_t[e];
     draw = run.spill_draw[e];
-    mark = run.spill_mark[e];
     i = run.spill_i[e] & 0x7fffffffu;
-    capped = (run.spill_i[e] >> 31) != 0u;
+    dead = (run.spill_i[e] >> 31) != 0u; // by the cap, before the hand-off (already counted)
+    if (Net::kRangeFlag == REBOP_FLAG_EXACT && draw - run.spill_mark[e] >= REBOP_DRAWS_PER_CHECK)
+      acc.flags |= REBOP_FLAG_EXACT;
   } else if (run.st_x) {
     net.load_state(x, run.st_x + jl, n);
     t = run.st_t[jl];
     draw = run.st_draw[jl];
-    mark = draw;
   } else {
     net.load_x0(x, run.x0_div ? run.x0 + (jl / run.x0_div) * net.S() : run.x0);
     t = 0.0;
     draw = 0;
-    mark = 0;
   }
   if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
   const uint64_t draw0 = draw;
+  const uint32_t i0 = i;
   // the cap counts from the trajectory's draws at the start of this call
   // (a resumed tail entry started it in the persistent launch)
   const uint64_t dlim =
       cap_limit(run, run.resume ? (run.st_x ? run.st_draw[jl] : 0ull) : draw);
   double Tc = GridLds ? 0.0 : grid_time(run, i), tot = 0.0;
-  int64_t *orec = run.out && lead ? run.out + jl + (uint64_t)i * Sn : nullptr;
-  bool done = false;
-  auto props_now = [&]() {
-    tot = net.props(x, cum);
+  const bool writes = run.out && lead;
+  // the draws and the grid position when the trajectory was absorbed
+  uint64_t end_draw = draw;
+  uint32_t end_i = i;
+  // some total of the wave was positive but not a usual one
+  bool odd = false;
+  auto absorb = [&](uint64_t d) {
+    dead = true;
+    tot = 0.0;
+    end_draw = d;
+    end_i = i;
+  };
+  // a new total that is not a usual one, after d draws
+  auto unusual = [&](uint64_t d) {
     if (tot == __builtin_inf()) {
       acc.flags |= REBOP_FLAG_RANGE;
       tot = 0.0;
     }
+    if (!(0.0 < tot)) absorb(d);
   };
-  props_now();
-  if (capped) tot = 0.0; // stopped by the cap before the hand-off (already counted)
+  if (!dead) {
+    tot = net.props(x, cum);
+    if (!usual_total(tot)) unusual(draw);
+  }
+  odd = __ballot(!dead && !usual_total(tot)) != 0ull;
+  bool finished = false;
+  auto finish = [&](uint64_t d) { // after d draws, if not absorbed before
+    if (!dead) absorb(d);
+    finished = true;
+    if (lead) {
+      if (run.final_x) net.write_counts(x, run.final_x + jl, n);
+      if (run.st_x) {
+        net.store_state(x, run.st_x + jl, n);
+        run.st_t[jl] = t;
+        run.st_draw[jl] = end_draw;
+      }
+      acc.events += (end_draw - draw0) - (end_i - i0);
+      acc.draws += end_draw - draw0;
+      acc.trajectories += 1;
+    }
+  };
+  // the straight rounds' stores: 32-bit indices into run.out, and a lane that
+  // writes nothing has one that the buffer's bounds check drops
+  constexpr uint32_t kDrop = 0x80000000u;
+  const uint32_t row = (uint32_t)Sn;
+  const WordBuffer out = word_buffer(run.out, FAST && run.out ? (nb + 1u) * row : 0u);
 
   // this lane's draw of the next round: ln reduced and its table row read,
   // the rest of the ln evaluated when the round starts
@@ -541,61 +677,108 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
     u_next = rebop_unif_of(blk);
   };
   fetch(draw);
-  while (!done) {
-    const double e_own = -rebop_ln64_finish(pre), u_own = u_next;
+  while (__ballot(i <= nb) != 0ull) {
+    double e_own = -rebop_ln64_finish(pre), u_own = u_next;
     const uint64_t d0 = draw;
+    if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
+    if (FAST && !odd) {
+      double xs[Net::MS], ts = t, tots = tot, T = grid_lds[i], Tn = grid_lds[i + 1u];
 #pragma unroll
+      for (int s = 0; s < Net::MS; ++s) xs[s] = x[s];
+      const uint32_t is = i;
+      uint32_t at = (lead ? 0u : kDrop) + i * row + (uint32_t)jl, worst = 0;
+      fetch(d0 + K);
+      group_steps<K>([&](auto step) {
+        constexpr int q = decltype(step)::q;
+        const double e = group_read<K, q>(e_own);
+        const double u = group_read<K, q>(u_own);
+        const double tn = t + usual_quotient(e, tot);
+        const bool rec = !(tn <= T);
+        const uint32_t k = net.choose(x, cum, tot * u);
+        net.affect(x, rec ? (uint32_t)Net::MR : k);
+        t = rec ? T : tn;
+        const double total = net.props(x, cum);
+        tot = rec ? tot : total;
+        const uint32_t far = usual_distance(total);
+        const uint32_t seen = rec ? 0u : far;
+        worst = worst > seen ? worst : seen;
+        net.write_raw_buffer(x, out, rec ? at : kDrop, (uint32_t)n);
+        at += rec ? row : 0u;
+        T = rec ? Tn : T;
+        i += rec ? 1u : 0u;
+        Tn = grid_lds[i + 1u];
+      });
+      if (__builtin_expect(__ballot(worst >= kUsualSpan) == 0ull, 1)) {
+        const uint32_t past = i > nb ? i - nb - 1u : 0u; // samples past the last one
+        i -= past;
+        const bool last = i > nb && !finished;
+        if (__builtin_expect(__ballot(last) != 0ull, 0))
+          if (last) {
+            t = grid_lds[nb];
+            finish(d0 + (K - past));
+          }
+        draw = d0 + K;
+        continue;
+      }
+      // an event made a total that is not a usual one: the round again, step
+      // by step (what it stored is stored again)
+      t = ts;
+      tot = tots;
+      i = is;
+#pragma unroll
+      for (int s = 0; s < Net::MS; ++s) x[s] = xs[s];
+      (void)net.props(x, cum);
+      // (the draws again too: kept, they would cost the straight round registers)
+      fetch(d0);
+      e_own = -rebop_ln64_finish(pre);
+      u_own = u_next;
+    }
+    int64_t *orec = run.out + jl + (uint64_t)i * Sn;
+#pragma unroll(K <= 4 ? K : 1)
     for (int q = 0; q < K; ++q) {
       const double e = group_read<K>(e_own, q);
       const double u = group_read<K>(u_own, q);
-      if (!done) {
-        const double T = GridLds ? grid_lds[i] : Tc; // i <= nb until done
-        // an absorbing (or capped) state takes no draw and records; the
-        // quotient is then unused (E / 0 is not trapped)
-        const bool live = 0.0 < tot;
-        const double tn = t + e / tot;
-        const bool rec = !live || tn > T;
-        draw += live ? 1u : 0u;
-        ov += (live && rec) ? 1u : 0u;
-        if (rec) {
-          if (orec) {
-            net.write_raw(x, orec, n);
-            orec += Sn;
-          }
-          if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
-          if (Net::kRangeFlag == REBOP_FLAG_EXACT && draw - mark >= REBOP_DRAWS_PER_CHECK)
-            acc.flags |= REBOP_FLAG_EXACT;
-          mark = draw;
-          t = T;
-          i += 1;
-          if constexpr (!GridLds) Tc = grid_time(run, i);
-          if (i > nb) {
-            if (lead && run.final_x) net.write_counts(x, run.final_x + jl, n);
-            if (lead && run.st_x) {
-              net.store_state(x, run.st_x + jl, n);
-              run.st_t[jl] = t;
-              run.st_draw[jl] = draw;
-            }
-            if (lead) {
-              acc.events += (draw - draw0) - ov;
-              acc.draws += draw - draw0;
-              acc.trajectories += 1;
-            }
-            done = true;
-          }
-        } else {
-          t = tn;
-          net.affect(x, net.choose(x, cum, tot * u));
-          props_now();
-          if constexpr (Net::kCap)
-            if (__builtin_expect(draw >= dlim, 0)) tot = hit_cap(run, acc, lead);
+      const double T = GridLds ? grid_lds[i] : Tc; // i <= nb + 1
+      double dt = usual_quotient(e, tot);
+      if (__builtin_expect(odd, 0))
+        if (!dead && !usual_total(tot)) dt = e / tot;
+      const double tn = t + dt;
+      // (a sample time is NaN only with an infinite horizon, which has a cap)
+      const bool rec = Net::kCap ? dead || tn > T : !(tn <= T);
+      const uint32_t k = net.choose(x, cum, tot * u);
+      net.affect(x, rec ? (uint32_t)Net::MR : k);
+      t = rec ? T : tn;
+      const double total = net.props(x, cum);
+      tot = rec ? tot : total;
+      const bool strange = !rec && !usual_total(total);
+      if (__builtin_expect(__ballot(strange) != 0ull, 0)) {
+        if (strange) unusual(d0 + q + 1);
+        odd = odd || __ballot(strange && !dead) != 0ull;
+      }
+      if constexpr (Net::kCap)
+        if (__builtin_expect(!rec && !dead && d0 + q + 1 >= dlim, 0)) {
+          (void)hit_cap(run, acc, lead);
+          absorb(d0 + q + 1);
         }
+      const bool sample = rec && i <= nb;
+      if (sample && writes) {
+        net.write_raw(x, orec, n);
+        orec += Sn;
+      }
+      i += sample ? 1u : 0u;
+      if constexpr (!GridLds)
+        if (sample) Tc = grid_time(run, i);
+      const bool last = sample && i > nb;
+      if (__builtin_expect(__ballot(last) != 0ull, 0)) {
+        if (last) finish(d0 + q + 1);
       }
       // after the first event's sample-time read, so that waiting for that
       // read does not wait for these
       if (q == 0) fetch(d0 + K);
     }
+    draw = d0 + K; // of a trajectory not yet absorbed
   }
+  if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
   return acc;
 }
 
@@ -682,8 +865,16 @@ __device__ __forceinline__ LaneTotals lane_events(Net &net, const rebop_dev_run 
 // using block q for its q-th event (read from lane q by DPP) -- each event
 // takes the next draw and an absorbing state takes none, so the blocks of a
 // round are used in order or not at all (the argument of lane_loop_group).
-// All lanes hold the same state; lane 0 of the group writes and counts.
-template <class Net, int K>
+// All lanes hold the same state; lane 0 of the group writes and counts.  As
+// there, an iteration has one path for every trajectory: an absorbed one
+// (total 0, quotient NaN) moves its time to infinity, and one that has ended
+// takes no jump and keeps its time.  Straight rounds have no branch: an ended
+// trajectory writes its last record again, and a round is done again step by
+// step if a total in it was not a usual one.  A wave takes the step-by-step
+// round while a trajectory has an absorbed state to report or records for
+// less than a round left.  WRITE: run.rec_offsets is set.  10^4 SIR
+// trajectories, both passes: 1152 us with branches, 940 us.
+template <class Net, int K, bool WRITE>
 __device__ __forceinline__ LaneTotals lane_events_group(Net &net, const rebop_dev_run &run, uint64_t gtid,
                                                         const double (*ln_tab)[4]) {
   LaneTotals acc;
@@ -701,53 +892,151 @@ __device__ __forceinline__ LaneTotals lane_events_group(Net &net, const rebop_de
   net.start(run, jl);
   net.load_x0(x, run.x0_div ? run.x0 + (jl / run.x0_div) * S : run.x0);
   if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
-  const bool write = run.rec_offsets != nullptr;
-  const uint64_t base = write ? run.rec_offsets[jl] : 0ull;
-  const uint64_t cap = write ? run.n_records[jl] : 0ull;
-  double t = 0.0;
+  const uint64_t base = WRITE ? run.rec_offsets[jl] : 0ull;
+  // the caller's count bounds the writes (see lane_events)
+  uint64_t room = WRITE ? run.n_records[jl] : 0ull; // records still to write
+  double *rt = run.rec_times + base;
+  int64_t *rs = run.rec_states + base * S;
+  const double tmax = run.tmax;
+  double t = 0.0, tot = 0.0;
   uint64_t draw = 0, rec = 0;
   const uint64_t dlim = cap_limit(run, 0ull);
-  bool stop = false; // the draw cap was reached
+  bool dead = false; // absorbed: tot is 0
+  bool odd = false;  // some total of the wave was positive but not a usual one
   auto emit = [&]() {
-    if (write && lead && rec < cap) {
-      run.rec_times[base + rec] = t;
-      net.write_counts(x, run.rec_states + (base + rec) * S, 1);
+    if (room != 0ull) {
+      room -= 1;
+      if (lead) {
+        *rt = t;
+        net.write_counts(x, rs, 1);
+      }
+      rt += 1;
+      rs += S;
     }
-    rec += 1;
   };
+  auto unusual = [&]() {
+    if (tot == __builtin_inf()) {
+      acc.flags |= REBOP_FLAG_RANGE; // time would stop (E / tot == 0)
+      tot = 0.0;
+    }
+    if (!(0.0 < tot)) {
+      dead = true;
+      tot = 0.0;
+    }
+  };
+  bool more = t < tmax;
+  if (more) {
+    tot = net.props(x, cum);
+    if (!usual_total(tot)) unusual();
+  }
+  odd = __ballot(more && !dead && !usual_total(tot)) != 0ull;
   emit();
-  while (t < run.tmax && !stop) {
-    const rebop_u32x4 blk = rebop_draw_block(run.seed, run.traj_begin + jl, draw + sub);
-    const double e_own = rebop_exp1_of_tab(blk, ln_tab), u_own = rebop_unif_of(blk);
+  rec = 1;
+  rebop_ln_pre pre;
+  double u_next;
+  auto fetch = [&](uint64_t d) {
+    const rebop_u32x4 blk = rebop_draw_block(run.seed, run.traj_begin + jl, d + sub);
+    pre = rebop_ln64_begin(rebop_u01_open_closed(blk.w[0], blk.w[1]), ln_tab);
+    u_next = rebop_unif_of(blk);
+  };
+  fetch(0);
+  uint64_t d0 = 0;
+  while (__ballot(more) != 0ull) {
+    double e_own = -rebop_ln64_finish(pre), u_own = u_next;
+    fetch(d0 + K);
+    if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
+    // an ended trajectory has a record to write again, the first at least
+    const bool careful = (more && (dead || (WRITE && room < (uint64_t)K))) ||
+                         (WRITE && (!net.small(x) || run.n_records[jl] == 0ull));
+    if (!Net::kCap && !odd && __ballot(careful) == 0ull) {
+      double xs[Net::MS], ts = t, tots = tot;
+#pragma unroll
+      for (int s = 0; s < Net::MS; ++s) xs[s] = x[s];
+      uint32_t fired = 0, worst = 0;
+      double *wt = rt - 1; // the last record written
+      int64_t *ws = rs - S;
+#pragma unroll
+      for (int q = 0; q < K; ++q) {
+        const double e = group_read<K>(e_own, q);
+        const double u = group_read<K>(u_own, q);
+        const double tn = t + usual_quotient(e, tot);
+        const uint32_t k = net.choose(x, cum, tot * u);
+        const bool on = t < tmax;
+        net.affect(x, on ? k : (uint32_t)Net::MR);
+        t = on ? tn : t;
+        tot = net.props(x, cum);
+        const uint32_t step = on ? 1u : 0u, far = usual_distance(tot);
+        fired += step;
+        const uint32_t seen = t < tmax ? far : 0u;
+        worst = worst > seen ? worst : seen;
+        if constexpr (WRITE) {
+          wt += step;
+          ws += step * S;
+          *wt = t;
+          net.write_small(x, ws);
+        }
+      }
+      if (__builtin_expect(__ballot(worst >= kUsualSpan) == 0ull, 1)) {
+        draw += fired;
+        rec += fired;
+        more = t < tmax;
+        if constexpr (WRITE) {
+          room -= fired;
+          rt = wt + 1;
+          rs = ws + S;
+        }
+        d0 += K;
+        continue;
+      }
+      // the round again, step by step (what it wrote is written again)
+      t = ts;
+      tot = tots;
+#pragma unroll
+      for (int s = 0; s < Net::MS; ++s) x[s] = xs[s];
+      (void)net.props(x, cum);
+      fetch(d0);
+      e_own = -rebop_ln64_finish(pre);
+      u_own = u_next;
+      fetch(d0 + K);
+    }
 #pragma unroll
     for (int q = 0; q < K; ++q) {
       const double e = group_read<K>(e_own, q);
       const double u = group_read<K>(u_own, q);
-      if (t < run.tmax && !stop) {
-        const double tot = net.props(x, cum);
-        if (!(0.0 < tot)) {
-          t = __builtin_inf();
-        } else if (tot == __builtin_inf()) {
-          acc.flags |= REBOP_FLAG_RANGE; // time would stop (E / tot == 0)
-          t = __builtin_inf();
-        } else {
-          draw += 1;
-          t = t + e / tot;
-          net.affect(x, net.choose(x, cum, tot * u));
-          if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
-          if constexpr (Net::kCap) {
-            if (__builtin_expect(draw >= dlim, 0)) {
-              hit_cap(run, acc, lead);
-              stop = true;
-            }
-          }
+      double dt = usual_quotient(e, tot);
+      if (__builtin_expect(odd, 0))
+        if (!dead && !usual_total(tot)) dt = e / tot;
+      // the time of an absorbed trajectory: infinity in place of NaN
+      const double tn = __builtin_fmin(t + dt, __builtin_inf());
+      const bool fires = more && !dead;
+      const uint32_t k = net.choose(x, cum, tot * u);
+      net.affect(x, fires ? k : (uint32_t)Net::MR);
+      t = more ? tn : t;
+      draw += fires ? 1u : 0u;
+      const double total = net.props(x, cum);
+      tot = fires ? total : tot;
+      rec += more ? 1u : 0u;
+      const bool was = more;
+      more = more && t < tmax;
+      if constexpr (Net::kCap)
+        if (__builtin_expect(fires && draw >= dlim, 0)) {
+          hit_cap(run, acc, lead);
+          more = false; // the draw cap was reached
         }
-        emit();
+      // (a total that no event will use is not looked at)
+      const bool strange = more && fires && !usual_total(total);
+      if (__builtin_expect(__ballot(strange) != 0ull, 0)) {
+        if (strange) unusual();
+        odd = odd || __ballot(strange && !dead) != 0ull;
       }
+      if (WRITE)
+        if (was) emit();
     }
+    d0 += K;
   }
+  if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
   if (lead) {
-    if (!write) run.n_records[jl] = rec;
+    if (!WRITE) run.n_records[jl] = rec;
     else if (run.n_records[jl] != rec) acc.flags |= REBOP_FLAG_RANGE;
     acc.events += draw;
     acc.draws += draw;

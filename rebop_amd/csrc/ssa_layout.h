@@ -40,6 +40,9 @@
  * below this (at most 16 KB per workgroup); above it they read the table in
  * global memory (grouped kernels: compute them) */
 #define REBOP_GRID_LDS 2048u
+/* NaNs after the LDS copy of the sample times in a grouped launch, which
+ * reads up to a round (16 draws) past a trajectory's last sample */
+#define REBOP_GRID_PAD 24u
 
 /* error flags raised by kernels */
 #define REBOP_FLAG_RANGE 1u
@@ -129,6 +132,30 @@ typedef struct {
   uint32_t *spill_i;    /* [cap] next grid point; bit 31: stopped by the draw cap */
   double *spill_x;      /* [S][cap] counts */
 } rebop_dev_run;
+
+#ifdef __cplusplus
+namespace rebop {
+/* The sample times of a grid or target run. */
+#if defined(__HIPCC__) || defined(__HIPCC_RTC__)
+__host__ __device__
+#endif
+inline uint64_t run_samples(const rebop_dev_run &run) {
+  return run.mode == REBOP_MODE_TARGET ? 1u : run.nb_steps + 1u;
+}
+/* Whether a grouped launch over S species may take straight rounds: the sample
+ * times fit LDS, and the stores' 32-bit indices, which run a round past the
+ * output, stay below 2^31 (and a sample's counts below 2^32 bytes). */
+#if defined(__HIPCC__) || defined(__HIPCC_RTC__)
+__host__ __device__
+#endif
+inline bool group_straight(const rebop_dev_run &run, uint32_t S) {
+  const uint64_t n = run_samples(run);
+  return run.mode != REBOP_MODE_EVENTS && n <= REBOP_GRID_LDS &&
+         (!run.out || ((n + REBOP_GRID_PAD) * run.n_traj < 0x80000000ull / (S ? S : 1u) &&
+                       run.n_traj < 0x20000000ull / (S ? S : 1u)));
+}
+} // namespace rebop
+#endif
 
 /*
  * One network of an LDS-kernel launch (a "job"), read at wave-uniform

@@ -665,7 +665,8 @@ __device__ __forceinline__ double item_feature(const ItemInputs &v, const double
 // Four threads per item: thread q computes logs 2q and 2q + 1 (of seven),
 // which the four share through LDS, and features 4q .. 4q+3.  A thread per
 // item took seven logarithms in a row on 16 workgroups and wrote its row two
-// bytes at a time (4096 items: 13.1 us, now 4.8 us).  wide: rows of X may be written eight bytes at a time.
+// bytes at a time (4096 items: 13.1 us, now 4.8 us).  wide: rows of X may be
+// written eight bytes at a time.
 __global__ void __launch_bounds__(256) features_kernel(int B, const uint32_t *__restrict__ item_point,
                                                        const uint32_t *__restrict__ item_sample,
                                                        const double *__restrict__ rates,
