@@ -550,8 +550,8 @@ __device__ __forceinline__ void group_steps(F &&f) {
 // trajectory's above all) are noticed at the end of the round, which is then
 // done again with the tests (the stores are the same).  10^4 SIR
 // trajectories of 250 samples, a call: 636 us with both paths branched over,
-// 557 us with one path and the tests, 488 us in straight rounds (59 vector
-// instructions an iteration with four lanes, 51 with sixteen).
+// 557 us with one path and the tests, 490 us in straight rounds (59 vector
+// instructions of straight code an iteration with four lanes, 51 with sixteen).
 //
 // Memory latency stays off the chain: `ln_tab` is the workgroup's LDS copy of
 // the ln table, whose rows for the next round's draws are read while this
