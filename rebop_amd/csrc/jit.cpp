@@ -254,22 +254,21 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "  for (uint32_t w = threadIdx.x; w < 512u; w += blockDim.x)\n";
   s += "    (&ln_lds[0][0])[w] = (&rebop_ln_table[0][0])[w];\n";
   s += "  const uint64_t samples = rebop::run_samples(run);\n";
-  s += "  const bool lds_grid = run.mode != REBOP_MODE_EVENTS && run.grid && samples <= REBOP_GRID_LDS;\n";
+  s += "  const bool lds_grid = run.grid && rebop::group_straight(run, " + Ss + ");\n";
   s += "  if (lds_grid)\n";
   s += "    for (uint32_t w = threadIdx.x; w < samples; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
   s += "  if (lds_grid && threadIdx.x < REBOP_GRID_PAD) grid_lds[samples + threadIdx.x] = __builtin_nan(\"\");\n";
   s += "  __syncthreads();\n";
-  s += "  const bool straight = rebop::group_straight(run, " + Ss + ");\n";
   s += "  JitNet<false> net;\n";
   s += "  const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
   s += "  rebop::LaneTotals acc;\n";
   // (a launch with 16 lanes is always one of straight rounds)
-  s += "  if constexpr (K == 16) acc = rebop::lane_loop_group<JitNet<false>, K, true, true>(net, run, gtid, ln_lds, grid_lds);\n";
+  s += "  if constexpr (K == 16) acc = rebop::lane_loop_group<JitNet<false>, K, true>(net, run, gtid, ln_lds, grid_lds);\n";
   s += "  else acc = run.mode == REBOP_MODE_EVENTS\n";
   s += "          ? (run.rec_offsets ? rebop::lane_events_group<JitNet<false>, K, true>(net, run, gtid, ln_lds)\n";
   s += "                             : rebop::lane_events_group<JitNet<false>, K, false>(net, run, gtid, ln_lds))\n";
-  s += "      : lds_grid && straight ? rebop::lane_loop_group<JitNet<false>, K, true, true>(net, run, gtid, ln_lds, grid_lds)\n";
-  s += "                             : rebop::lane_loop_group<JitNet<false>, K, false, false>(net, run, gtid, ln_lds, nullptr);\n";
+  s += "      : lds_grid ? rebop::lane_loop_group<JitNet<false>, K, true>(net, run, gtid, ln_lds, grid_lds)\n";
+  s += "                 : rebop::lane_loop_group<JitNet<false>, K, false>(net, run, gtid, ln_lds, nullptr);\n";
   s += "  rebop::flush_totals(acc, run, blk_ctr);\n";
   s += "}\n";
   // REBOP_JIT_WAVES_PER_EU=<n>: ask the compiler to fit n waves per SIMD in

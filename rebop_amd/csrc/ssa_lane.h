@@ -560,13 +560,13 @@ __device__ __forceinline__ void group_steps(F &&f) {
 // `grid_lds` its LDS copy of the sample times, followed by REBOP_GRID_PAD
 // NaNs, read an iteration ahead.  No vector-memory wait is left
 // in the loop, so the sample stores are never waited for.  GridLds: grid_lds
-// holds the sample times (else the next one is carried, computed at each
-// sample, for grids too long for LDS).
-template <class Net, int K, bool GridLds, bool Straight>
+// holds the sample times and group_straight holds for the run (else the next
+// sample time is carried, computed at each sample).
+template <class Net, int K, bool GridLds>
 __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_run &run,
                                                       uint64_t gtid, const double (*ln_tab)[4],
                                                       const double *grid_lds) {
-  constexpr bool FAST = GridLds && Straight && !Net::kCap;
+  constexpr bool FAST = GridLds && !Net::kCap;
   LaneTotals acc;
   const uint64_t n = run.n_traj;
   const uint64_t e = gtid / K; // group index
