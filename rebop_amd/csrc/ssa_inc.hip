@@ -12,13 +12,19 @@
 // one that a rounding could turn is made again the reference's way:
 //
 // - Propensities enter the sums quantised: q_r = rint(a_r / g), g a power of
-//   two chosen so that the total Q = sum q_r lies in [2^49, 2^53).  Sums of
-//   such integers are exact in binary64 whatever their order, so nothing
-//   drifts.  When Q leaves the range the sums are rebuilt with another g.
+//   two chosen so that the total Q = sum q_r lies in [2^48, 2^52).  An event's
+//   differences are added one by one, so on the way a sum holds old and new
+//   values at once: at most Q_old + Q_new, below 2^53 while both totals are
+//   in the range.  Integers up to there are exact in binary64 whatever the
+//   order of the additions, so nothing drifts.  (Where Q_new is not in the
+//   range, an addition can lose a unit only above 2^53, at most
+//   Q_old + Q_new - 2^53 < Q_new - 2^52 units in all, so the total found is
+//   not in the range either.)  When Q leaves it the sums are rebuilt with
+//   another g.
 // - The reference's partial sum cum_r and g Q_r differ by at most
 //   R/2 g + R 2^-53 g Q (quantisation; R rounded additions of non-negative
-//   terms), which is below 16 R 2^-53 of the total and below (3/2) R units of
-//   g.  kKappa and epsilon below are these bounds with room to spare.
+//   terms), which is at most 17 R 2^-53 of the total and below R units of g.
+//   kappa and eps below are these bounds with room to spare.
 // - The time is kept as an interval [tl, th] that holds the reference's t:
 //   both ends take fl(end + E/total (1 -+ kappa)), and rounding is monotone.
 //   A comparison with a sample time that the interval straddles is not
@@ -33,7 +39,7 @@
 //   total outside [1e-200, 1e200].
 //
 // With 512 reactions, 5e4 events and 200 samples a trajectory restarts with a
-// probability of about 1e-7 and a choice is repeated about once in 1e9 events.
+// probability of about 2e-7 and a choice is repeated about once in 1e9 events.
 //
 // Layout: a wave runs eight trajectories, eight lanes each.  The lanes of a
 // group hold the same scalar state; they share the draws (lane j computes the
@@ -66,8 +72,10 @@ namespace rebop {
 constexpr uint32_t kIncGroup = 8; // lanes per trajectory
 constexpr uint32_t kIncTraj = 64 / kIncGroup; // trajectories per wave
 
-// The total is kept in [kIncLo, kIncHi) units; a rebuild puts it in [2^51, 2^52).
-constexpr double kIncLo = 0x1p49, kIncHi = 0x1p53;
+// The total is kept in [kIncLo, kIncHi) units; a rebuild puts it in
+// [2^kIncTarget, 2^(kIncTarget + 1)).
+constexpr double kIncLo = 0x1p48, kIncHi = 0x1p52;
+constexpr int32_t kIncTarget = 50;
 
 // LDS of one wave, in bytes from its start: the draws [8][8] (E, U), a row of
 // propensities per group for the sequential sums, the sums, then (STORE) the
@@ -254,8 +262,8 @@ struct IncNet {
     }
     if (!(s > 1e-200 && s < 1e200)) return false;
     const int32_t e = (int32_t)(rebop_f64_bits(s) >> 52) - 1023;
-    g = rebop_pow2i(e - 51);
-    inv_g = rebop_pow2i(51 - e);
+    g = rebop_pow2i(e - kIncTarget);
+    inv_g = rebop_pow2i(kIncTarget - e);
     const uint32_t ns = 8u + ((((R - 1u) >> bsh) >> 3) + 1u) * 8u;
     for (uint32_t i = j; i < ns; i += kIncGroup) sums[i] = 0.0;
     inc_sync();
@@ -382,7 +390,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(EXPR ? 
     net.tok = (inc_g4_t)(const void *)job.inc_tok;
     net.eps = 4.0 * (double)job.R + 8.0;
     net.inv_g = net.g = 0.0;
-    const double kappa = (16.0 * (double)job.R + 16.0) * 0x1p-53;
+    const double kappa = (32.0 * (double)job.R + 32.0) * 0x1p-53;
     const uint64_t n = job.n_traj;
     const uint32_t nb = (uint32_t)job.nb_steps;
     const uint64_t Sn = (uint64_t)job.S * n;
