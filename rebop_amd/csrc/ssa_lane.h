@@ -624,7 +624,7 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
   // the draws and the grid position when the trajectory was absorbed
   uint64_t end_draw = draw;
   uint32_t end_i = i;
-  // some total of the wave was positive but not a usual one
+  // some total of the wave was positive but not a usual one, or a time NaN
   bool odd = false;
   auto absorb = [&](uint64_t d) {
     dead = true;
@@ -644,7 +644,9 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
     tot = net.props(x, cum);
     if (!usual_total(tot)) unusual(draw);
   }
-  odd = __ballot(!dead && !usual_total(tot)) != 0ull;
+  // (a batch's time may have been set to NaN, which no sample time is before:
+  // events until the state is absorbed, as with one lane)
+  odd = __ballot(!dead && (!usual_total(tot) || t != t)) != 0ull;
   bool finished = false;
   auto finish = [&](uint64_t d) { // after d draws, if not absorbed before
     if (!dead) absorb(d);
@@ -744,7 +746,9 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
         if (!dead && !usual_total(tot)) dt = e / tot;
       const double tn = t + dt;
       // (a sample time is NaN only with an infinite horizon, which has a cap)
-      const bool rec = Net::kCap ? dead || tn > T : !(tn <= T);
+      bool rec = Net::kCap ? dead || tn > T : !(tn <= T);
+      if constexpr (!Net::kCap)
+        if (__builtin_expect(odd, 0)) rec = dead || tn > T; // t may be NaN
       const uint32_t k = net.choose(x, cum, tot * u);
       net.affect(x, rec ? (uint32_t)Net::MR : k);
       t = rec ? T : tn;

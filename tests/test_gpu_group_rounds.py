@@ -82,3 +82,23 @@ def test_every_event_recorded(spec, tmax, n):
     for j in range(n):
         t, x = o.run_all_events(23, 5 + j, spec[2], tmax)
         assert np.array_equal(ts[j].view(np.uint64), t.view(np.uint64)) and np.array_equal(xs[j], x), j
+
+
+@pytest.mark.parametrize("n", [3, 64, 4100, 40_000])
+def test_a_time_set_to_nan_fires_until_absorbed(n):
+    """No sample time is before NaN, so such a trajectory runs on to its
+    absorbing state, whatever the lanes per trajectory (16, 4, 2, 1)."""
+    b = build_device(DECAY(9), 23).batch(n, traj_begin=5)
+    t = np.zeros(n)
+    t[::3] = np.nan
+    b.set_time(t)
+    b.advance_until(0.7)
+    x, time, draws = b.get_species(), b.get_time(), b.get_draws()
+    assert np.array_equal(x[::3], np.tile([0, 9], (len(x[::3]), 1)))
+    assert np.array_equal(draws[::3], np.full(len(draws[::3]), 9))
+    assert np.array_equal(time, np.full(n, 0.7))
+    o = build_oracle(DECAY(9))
+    for j in range(1, min(n, 60), 3):  # the others of the same waves
+        w = o.state(DECAY(9)[2], 23, traj=5 + j)
+        w.advance_until(0.7)
+        assert np.array_equal(x[j], w.x) and draws[j] == w.draws, j
