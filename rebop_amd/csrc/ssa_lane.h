@@ -612,6 +612,9 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
     t = 0.0;
     draw = 0;
   }
+  // a batch's time may have been set to NaN, which is past no sample time:
+  // events until the state is absorbed, as from minus infinity
+  if (t != t) t = -__builtin_inf();
   if (!net.in_range(x)) acc.flags |= Net::kRangeFlag;
   const uint64_t draw0 = draw;
   const uint32_t i0 = i;
@@ -624,7 +627,7 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
   // the draws and the grid position when the trajectory was absorbed
   uint64_t end_draw = draw;
   uint32_t end_i = i;
-  // some total of the wave was positive but not a usual one, or a time NaN
+  // some total of the wave was positive but not a usual one
   bool odd = false;
   auto absorb = [&](uint64_t d) {
     dead = true;
@@ -644,9 +647,7 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
     tot = net.props(x, cum);
     if (!usual_total(tot)) unusual(draw);
   }
-  // (a batch's time may have been set to NaN, which no sample time is before:
-  // events until the state is absorbed, as with one lane)
-  odd = __ballot(!dead && (!usual_total(tot) || t != t)) != 0ull;
+  odd = __ballot(!dead && !usual_total(tot)) != 0ull;
   bool finished = false;
   auto finish = [&](uint64_t d) { // after d draws, if not absorbed before
     if (!dead) absorb(d);
@@ -746,9 +747,7 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
         if (!dead && !usual_total(tot)) dt = e / tot;
       const double tn = t + dt;
       // (a sample time is NaN only with an infinite horizon, which has a cap)
-      bool rec = Net::kCap ? dead || tn > T : !(tn <= T);
-      if constexpr (!Net::kCap)
-        if (__builtin_expect(odd, 0)) rec = dead || tn > T; // t may be NaN
+      const bool rec = Net::kCap ? dead || tn > T : !(tn <= T);
       const uint32_t k = net.choose(x, cum, tot * u);
       net.affect(x, rec ? (uint32_t)Net::MR : k);
       t = rec ? T : tn;
