@@ -232,9 +232,13 @@ int rebop_system_add_reaction(rebop_gillespie *g, double rate, const uint32_t *r
 
 /* Uploads the network to the current device and compiles (cached) the
  * kernel `kernel` (REBOP_KERNEL_*; AUTO: the one an AUTO run would use) for
- * it, so that the first run does not pay for them.  Without a device it only
- * compiles, which checks the specialised kernel for gfx950.  No counterpart
- * in the reference (which has no device code to prepare). */
+ * it, so that the first run does not pay for them.  A specialised kernel is
+ * compiled in the forms that grid and target runs of any size take; its forms
+ * for rate tables and for recording every event with several lanes per
+ * trajectory are compiled by the first call that takes them, as is every form
+ * of a network that was not prepared.  Without a device it only compiles,
+ * which checks the specialised kernel for gfx950.  No counterpart in the
+ * reference (which has no device code to prepare). */
 int rebop_gillespie_prepare(const rebop_gillespie *g, int kernel);
 
 /* The autotuner's choice: which kernel and launch shape AUTO runs. */

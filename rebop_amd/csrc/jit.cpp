@@ -218,13 +218,15 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   // The ln table and (plain grid runs with nb_steps < REBOP_GRID_LDS) the
   // sample times are read from LDS copies, so that no event waits on vector
   // memory (such a wait also waits for the lane's earlier sample stores).
-  s += "template <bool SWEEP>\n__device__ __forceinline__ void jit_body(const rebop_dev_run &run) {\n";
-  s += "  __shared__ unsigned long long blk_ctr[4];\n";
-  s += "  __shared__ double ln_lds[128][4];\n";
-  s += "  extern __shared__ double grid_lds[];\n";
-  s += "  if (threadIdx.x < 4) blk_ctr[threadIdx.x] = 0ull;\n";
+  s += "struct JitLds { unsigned long long ctr[4]; double ln[128][4]; };\n";
+  s += "__device__ __forceinline__ void jit_begin(JitLds &l) {\n";
+  s += "  if (threadIdx.x < 4) l.ctr[threadIdx.x] = 0ull;\n";
   s += "  for (uint32_t w = threadIdx.x; w < 512u; w += blockDim.x)\n";
-  s += "    (&ln_lds[0][0])[w] = (&rebop_ln_table[0][0])[w];\n";
+  s += "    (&l.ln[0][0])[w] = (&rebop_ln_table[0][0])[w];\n}\n";
+  s += "template <bool SWEEP>\n__device__ __forceinline__ void jit_body(const rebop_dev_run &run) {\n";
+  s += "  __shared__ JitLds l;\n";
+  s += "  extern __shared__ double grid_lds[];\n";
+  s += "  jit_begin(l);\n";
   s += "  const bool lds_grid = !SWEEP && run.mode == REBOP_MODE_GRID && run.grid && run.nb_steps < REBOP_GRID_LDS;\n";
   s += "  if (lds_grid)\n";
   s += "    for (uint32_t w = threadIdx.x; w <= (uint32_t)run.nb_steps; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
@@ -235,42 +237,63 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "  if (lds_grid) {\n";
   s += "    JitNet<SWEEP, true> net;\n";
   s += "    net.gl = grid_lds;\n";
-  s += "    acc = rebop::lane_loop(net, run, gtid, nthreads, ln_lds);\n";
+  s += "    acc = rebop::lane_loop(net, run, gtid, nthreads, l.ln);\n";
   s += "  } else {\n";
   s += "    JitNet<SWEEP> net;\n";
-  s += "    acc = run.mode == REBOP_MODE_EVENTS ? rebop::lane_events(net, run, gtid, nthreads, ln_lds)\n";
-  s += "                                        : rebop::lane_loop(net, run, gtid, nthreads, ln_lds);\n";
+  s += "    acc = !SWEEP && run.mode == REBOP_MODE_EVENTS ? rebop::lane_events(net, run, gtid, nthreads, l.ln)\n";
+  s += "                                                  : rebop::lane_loop(net, run, gtid, nthreads, l.ln);\n";
   s += "  }\n";
-  s += "  rebop::flush_totals(acc, run, blk_ctr);\n";
+  s += "  rebop::flush_totals(acc, run, l.ctr);\n";
   s += "}\n";
-  // grouped kernels: the ln table and (nb_steps < REBOP_GRID_LDS) the sample
-  // times copied into LDS, so that the serial loop never waits on vector
-  // memory (the launch sizes the dynamic LDS for the sample times)
-  s += "template <int K>\n__device__ __forceinline__ void jit_body_group(const rebop_dev_run &run) {\n";
-  s += "  __shared__ unsigned long long blk_ctr[4];\n";
-  s += "  __shared__ double ln_lds[128][4];\n";
-  s += "  extern __shared__ double grid_lds[];\n";
-  s += "  if (threadIdx.x < 4) blk_ctr[threadIdx.x] = 0ull;\n";
-  s += "  for (uint32_t w = threadIdx.x; w < 512u; w += blockDim.x)\n";
-  s += "    (&ln_lds[0][0])[w] = (&rebop_ln_table[0][0])[w];\n";
-  s += "  const uint64_t samples = rebop::run_samples(run);\n";
-  s += "  const bool lds_grid = run.grid && rebop::group_straight(run, " + Ss + ");\n";
-  s += "  if (lds_grid)\n";
-  s += "    for (uint32_t w = threadIdx.x; w < samples; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
-  s += "  if (lds_grid && threadIdx.x < REBOP_GRID_PAD) grid_lds[samples + threadIdx.x] = __builtin_nan(\"\");\n";
+  // every event recorded, K lanes per trajectory
+  s += "template <int K, bool WRITE>\n__device__ __forceinline__ void jit_body_events(const rebop_dev_run &run) {\n";
+  s += "  __shared__ JitLds l;\n";
+  s += "  jit_begin(l);\n";
   s += "  __syncthreads();\n";
   s += "  JitNet<false> net;\n";
   s += "  const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
-  s += "  rebop::LaneTotals acc;\n";
-  // (a launch with 16 lanes is always one of straight rounds)
-  s += "  if constexpr (K == 16) acc = rebop::lane_loop_group<JitNet<false>, K, true>(net, run, gtid, ln_lds, grid_lds);\n";
-  s += "  else acc = run.mode == REBOP_MODE_EVENTS\n";
-  s += "          ? (run.rec_offsets ? rebop::lane_events_group<JitNet<false>, K, true>(net, run, gtid, ln_lds)\n";
-  s += "                             : rebop::lane_events_group<JitNet<false>, K, false>(net, run, gtid, ln_lds))\n";
-  s += "      : lds_grid ? rebop::lane_loop_group<JitNet<false>, K, true>(net, run, gtid, ln_lds, grid_lds)\n";
-  s += "                 : rebop::lane_loop_group<JitNet<false>, K, false>(net, run, gtid, ln_lds, nullptr);\n";
-  s += "  rebop::flush_totals(acc, run, blk_ctr);\n";
+  s += "  rebop::LaneTotals acc = rebop::lane_events_group<JitNet<false>, K, WRITE>(net, run, gtid, l.ln);\n";
+  s += "  rebop::flush_totals(acc, run, l.ctr);\n";
   s += "}\n";
+  // grouped kernels: the ln table and (GRID_LDS, a run with group_straight) the
+  // sample times copied into LDS, so that the serial loop never waits on
+  // vector memory (the launch sizes the dynamic LDS for the sample times)
+  s += "template <int K, bool GRID_LDS>\n__device__ __forceinline__ void jit_body_group(const rebop_dev_run &run) {\n";
+  s += "  __shared__ JitLds l;\n";
+  s += "  extern __shared__ double grid_lds[];\n";
+  s += "  jit_begin(l);\n";
+  s += "  if constexpr (GRID_LDS) {\n";
+  s += "    const uint64_t samples = rebop::run_samples(run);\n";
+  s += "    for (uint32_t w = threadIdx.x; w < samples; w += blockDim.x) grid_lds[w] = run.grid[w];\n";
+  s += "    if (threadIdx.x < REBOP_GRID_PAD) grid_lds[samples + threadIdx.x] = __builtin_nan(\"\");\n";
+  s += "  }\n";
+  s += "  __syncthreads();\n";
+  s += "  JitNet<false> net;\n";
+  s += "  const uint64_t gtid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;\n";
+  s += "  rebop::LaneTotals acc = rebop::lane_loop_group<JitNet<false>, K, GRID_LDS>(net, run, gtid, l.ln, grid_lds);\n";
+  s += "  rebop::flush_totals(acc, run, l.ctr);\n";
+  s += "}\n";
+  return s;
+}
+
+const char *jit_variant_name(int v) {
+  static const char *const names[kJitVariants] = {"main", "g2", "g4", "g16", "g2_far", "g4_far", "sweep",
+                                                  "ev2_count", "ev2_write", "ev4_count", "ev4_write"};
+  return names[v];
+}
+
+uint32_t jit_prepare_set(uint32_t R, bool cap) {
+  return jit_bit(kJitMain) | jit_bit(kJitG2) | jit_bit(kJitG4) | jit_bit(kJitG2Far) | jit_bit(kJitG4Far) |
+         (jit_sixteen(R, cap) ? jit_bit(kJitG16) : 0u);
+}
+
+// The entry points of the variants in `mask`, after jit_source's text.
+static std::string jit_kernels(uint32_t mask) {
+  static const char *const body[kJitVariants] = {
+      "jit_body<false>",           "jit_body_group<2, true>",   "jit_body_group<4, true>",
+      "jit_body_group<16, true>",  "jit_body_group<2, false>",  "jit_body_group<4, false>",
+      "jit_body<true>",            "jit_body_events<2, false>", "jit_body_events<2, true>",
+      "jit_body_events<4, false>", "jit_body_events<4, true>"};
   // REBOP_JIT_WAVES_PER_EU=<n>: ask the compiler to fit n waves per SIMD in
   // the main kernel's registers (a tuning knob; unset: the compiler's choice)
   std::string occ;
@@ -278,13 +301,11 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
     const long n = std::strtol(v, nullptr, 10);
     if (n >= 1 && n <= 8) occ = " __attribute__((amdgpu_waves_per_eu(" + std::to_string(n) + ")))";
   }
-  s += "extern \"C\" __global__ void __launch_bounds__(256)" + occ +
-       " rebop_ssa_jit(rebop_dev_run run) { jit_body<false>(run); }\n";
-  s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_sweep(rebop_dev_run run) { jit_body<true>(run); }\n";
-  s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g2(rebop_dev_run run) { jit_body_group<2>(run); }\n";
-  s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g4(rebop_dev_run run) { jit_body_group<4>(run); }\n";
-  if (!cap) // with a draw cap every round is stepped through, and long ones only cost code
-    s += "extern \"C\" __global__ void __launch_bounds__(256) rebop_ssa_jit_g16(rebop_dev_run run) { jit_body_group<16>(run); }\n";
+  std::string s;
+  for (int v = 0; v < kJitVariants; ++v)
+    if (mask & jit_bit(v))
+      s += "extern \"C\" __global__ void __launch_bounds__(256)" + (v == kJitMain ? occ : std::string()) +
+           " rebop_ssa_jit_" + jit_variant_name(v) + "(rebop_dev_run run) { " + body[v] + "(run); }\n";
   return s;
 }
 
@@ -420,69 +441,63 @@ static int compile(const std::string &src, std::vector<char> *code, std::string 
   return 0;
 }
 
-// Compiles (or finds in the cache) the kernel for `src` on the current device.
-int jit_get(const std::string &src, JitKernel *out, std::string *err) {
+// The code object of `src` from the disk cache, or compiled.
+static int code_object(const std::string &src, std::vector<char> *code, std::string *err) {
+  // REBOP_DUMP_SPECIALIZED=<file>: write the generated kernel source there
+  if (const char *path = std::getenv("REBOP_DUMP_SPECIALIZED")) write_file(path, src.data(), src.size());
+  if (disk_cache_get(src, code)) return 0;
+  if (int rc = compile(src, code, err)) return rc;
+  disk_cache_put(src, *code);
+  return 0;
+}
+
+// Loads the variants of `mask` that `out` does not hold for the network
+// `base`: from one module, compiled (or found in a cache) for the current
+// device.  `all`: the variants that are prepared together, whose module the
+// disk cache may hold.
+int jit_get(const std::string &base, uint32_t mask, uint32_t all, JitKernel *out, std::string *err) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess) {
     *err = "hipGetDevice failed";
     return -1;
   }
   std::lock_guard<std::mutex> lock(g_jit_mu);
-  auto key = std::make_pair(dev, src);
-  auto it = g_jit_cache.find(key);
-  if (it != g_jit_cache.end()) {
-    *out = it->second;
-    return 0;
+  JitKernel &k = g_jit_cache[std::make_pair(dev, base)];
+  uint32_t missing = mask & ~k.have();
+  if (missing) {
+    std::vector<char> code;
+    if (missing != all && (missing & ~all) == 0u && disk_cache_get(base + jit_kernels(all), &code))
+      missing = all & ~k.have();
+    else if (int rc = code_object(base + jit_kernels(missing), &code, err))
+      return rc;
+    hipModule_t mod = nullptr; // loaded until the process ends, as its functions may be in use
+    hipError_t he = hipModuleLoadData(&mod, code.data());
+    if (he != hipSuccess) {
+      *err = std::string("hipModuleLoadData: ") + hipGetErrorString(he);
+      return -1;
+    }
+    hipFunction_t fn[kJitVariants] = {};
+    for (int v = 0; v < kJitVariants && he == hipSuccess; ++v)
+      if (missing & jit_bit(v))
+        he = hipModuleGetFunction(&fn[v], mod, (std::string("rebop_ssa_jit_") + jit_variant_name(v)).c_str());
+    if (he != hipSuccess) {
+      *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(he);
+      return -1;
+    }
+    for (int v = 0; v < kJitVariants; ++v)
+      if (fn[v]) k.fn[v] = fn[v];
   }
-  std::vector<char> code;
-  if (!disk_cache_get(src, &code)) {
-    if (int rc = compile(src, &code, err)) return rc;
-    disk_cache_put(src, code);
-  }
-  JitKernel k;
-  hipError_t he = hipModuleLoadData(&k.mod, code.data());
-  if (he != hipSuccess) {
-    *err = std::string("hipModuleLoadData: ") + hipGetErrorString(he);
-    return -1;
-  }
-  he = hipModuleGetFunction(&k.fn, k.mod, "rebop_ssa_jit");
-  if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_sweep, k.mod, "rebop_ssa_jit_sweep");
-  if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_g2, k.mod, "rebop_ssa_jit_g2");
-  if (he == hipSuccess) he = hipModuleGetFunction(&k.fn_g4, k.mod, "rebop_ssa_jit_g4");
-  if (he == hipSuccess && src.find("rebop_ssa_jit_g16") != std::string::npos)
-    he = hipModuleGetFunction(&k.fn_g16, k.mod, "rebop_ssa_jit_g16");
-  if (he != hipSuccess) {
-    *err = std::string("hipModuleGetFunction: ") + hipGetErrorString(he);
-    return -1;
-  }
-  g_jit_cache.emplace(key, k);
   *out = k;
   return 0;
 }
 
-
-// Compiles `src` for gfx950 without loading it (usable without a device).
-int jit_compile_only(const std::string &src, size_t *code_size, std::string *err) {
-  hiprtcProgram prog;
-  hiprtcResult rr = hiprtcCreateProgram(&prog, src.c_str(), "rebop_ssa_jit.hip", kEmbeddedHeaderCount,
-                                        kEmbeddedHeaderSources, kEmbeddedHeaderNames);
-  if (rr != HIPRTC_SUCCESS) {
-    *err = hiprtcGetErrorString(rr);
-    return -1;
-  }
-  rr = hiprtcCompileProgram(prog, kNumCompileOptions, const_cast<const char **>(kCompileOptions));
-  if (rr != HIPRTC_SUCCESS) {
-    size_t ls = 0;
-    hiprtcGetProgramLogSize(prog, &ls);
-    std::string log(ls, '\0');
-    if (ls) hiprtcGetProgramLog(prog, &log[0]);
-    *err = log;
-    hiprtcDestroyProgram(&prog);
-    return -1;
-  }
-  hiprtcGetCodeSize(prog, code_size);
-  hiprtcDestroyProgram(&prog);
-  return 0;
+// Compiles the variants of `mask` for gfx950 without loading them (usable
+// without a device).
+int jit_compile_only(const std::string &base, uint32_t mask, std::string *err) {
+  const std::string src = base + jit_kernels(mask);
+  if (const char *path = std::getenv("REBOP_DUMP_SPECIALIZED")) write_file(path, src.data(), src.size());
+  std::vector<char> code;
+  return compile(src, &code, err);
 }
 
 size_t jit_dynamic_lds(const rebop_dev_run &run) {
@@ -493,16 +508,15 @@ size_t jit_dynamic_lds(const rebop_dev_run &run) {
   return samples <= REBOP_GRID_LDS ? sizeof(double) * (size_t)(samples + REBOP_GRID_PAD) : 0u;
 }
 
-hipError_t jit_occupancy(const JitKernel &k, int threads, size_t lds, int *blocks_per_cu) {
-  return hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k.fn, threads, lds);
+hipError_t jit_occupancy(const JitKernel &k, int variant, int threads, size_t lds, int *blocks_per_cu) {
+  return hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, k.fn[variant], threads, lds);
 }
 
-hipError_t jit_launch(const JitKernel &k, const rebop_dev_run &run, int blocks, int threads,
-                      hipStream_t stream, int group) {
+hipError_t jit_launch(const JitKernel &k, int variant, const rebop_dev_run &run, int blocks, int threads,
+                      hipStream_t stream) {
   rebop_dev_run arg = run;
   void *params[] = {&arg};
-  hipFunction_t f = run.rates ? k.fn_sweep : group == 16 ? k.fn_g16 : group == 4 ? k.fn_g4 : group == 2 ? k.fn_g2 : k.fn;
-  return hipModuleLaunchKernel(f, (unsigned)blocks, 1, 1, (unsigned)threads, 1, 1,
+  return hipModuleLaunchKernel(k.fn[variant], (unsigned)blocks, 1, 1, (unsigned)threads, 1, 1,
                                (unsigned)jit_dynamic_lds(run), stream, params, nullptr);
 }
 

@@ -26,31 +26,61 @@ struct JitReaction {
   std::vector<std::pair<uint32_t, uint32_t>> terms;
 };
 
+// The kernels of a network, each compiled when it is first launched or
+// prepared: a run uses one or two of them, and compiling all of them for the
+// first call made it wait 1.36 s (SIR) to 7.8 s (32 species, 64 reactions);
+// the one it launches takes 0.40 s to 0.99 s.  (Each compilation also parses
+// the headers, 0.35 s, so those prepared together are compiled together.)
+enum JitVariant {
+  kJitMain,     // one lane per trajectory
+  kJitG2,       // 2 lanes per trajectory (plain launches), runs with group_straight
+  kJitG4,       // 4 lanes per trajectory, also the tail of a persistent launch
+  kJitG16,      // 16 lanes per trajectory (jit_sixteen)
+  kJitG2Far,    // 2 and 4 lanes, runs without group_straight
+  kJitG4Far,
+  kJitSweep,    // one lane per trajectory, rate tables
+  kJitEv2Count, // every event recorded with 2 lanes: counting the records, then writing them
+  kJitEv2Write,
+  kJitEv4Count, // the same with 4 lanes
+  kJitEv4Write,
+  kJitVariants
+};
+constexpr uint32_t jit_bit(int variant) { return 1u << variant; }
+
 struct JitKernel {
-  hipModule_t mod = nullptr;
-  hipFunction_t fn = nullptr;
-  hipFunction_t fn_sweep = nullptr;
-  hipFunction_t fn_g2 = nullptr; // 2 lanes per trajectory (plain launches)
-  hipFunction_t fn_g4 = nullptr; // 4 lanes per trajectory
-  hipFunction_t fn_g16 = nullptr; // 16 lanes per trajectory (not with a draw cap)
+  hipFunction_t fn[kJitVariants] = {};
+  uint32_t have() const {
+    uint32_t m = 0;
+    for (int v = 0; v < kJitVariants; ++v) m |= fn[v] ? jit_bit(v) : 0u;
+    return m;
+  }
 };
 
-// Kernel source for a network of S species and the given reactions; with
-// `system`, the define_system arithmetic (integer mass-action products over
-// `terms`, first-match choice); with `cap`, the loops check the draw cap.
+// Whether a network of R reactions has the kernel with 16 lanes, whose round
+// of sixteen events is straight code.  The larger the network, the less of an
+// event its draw is, and the longer the code: 12 species and 24 reactions, one
+// trajectory 158 us with four lanes and 128 us with sixteen, 4096 178 and
+// 153 us; 20 and 40 308 and 298 us, 371 and 360 us; 32 and 64 672 and 664 us,
+// 746 and 769 us, with 6.6 s of compilation against 2.
+inline bool jit_sixteen(uint32_t R, bool cap) { return R <= 32u && !cap; }
+// The variants of a grid or target run of any size, which are prepared together.
+uint32_t jit_prepare_set(uint32_t R, bool cap);
+
+// Kernel source for a network of S species and the given reactions, without
+// the entry points; with `system`, the define_system arithmetic (integer
+// mass-action products over `terms`, first-match choice); with `cap`, the
+// loops check the draw cap.
 std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool system = false,
                        bool cap = false);
-// Compiles (or finds in the cache) and loads the kernel on the current device.
-int jit_get(const std::string &src, JitKernel *out, std::string *err);
+// Compiles (or finds in a cache) and loads variants on the current device.
+int jit_get(const std::string &base, uint32_t mask, uint32_t all, JitKernel *out, std::string *err);
 // Compiles for gfx950 without loading (no device needed).
-int jit_compile_only(const std::string &src, size_t *code_size, std::string *err);
+int jit_compile_only(const std::string &base, uint32_t mask, std::string *err);
 // Dynamic LDS bytes a launch of `run` takes (the LDS copy of the sample times).
 size_t jit_dynamic_lds(const rebop_dev_run &run);
-hipError_t jit_occupancy(const JitKernel &k, int threads, size_t lds, int *blocks_per_cu);
-// group = lanes per trajectory (1, 2, 4 or 16; above 1 only for plain, non-sweep
-// runs, 16 only without a draw cap)
-hipError_t jit_launch(const JitKernel &k, const rebop_dev_run &run, int blocks, int threads,
-                      hipStream_t stream, int group = 1);
+hipError_t jit_occupancy(const JitKernel &k, int variant, int threads, size_t lds, int *blocks_per_cu);
+hipError_t jit_launch(const JitKernel &k, int variant, const rebop_dev_run &run, int blocks, int threads,
+                      hipStream_t stream);
 
 } // namespace rebop
 

@@ -739,7 +739,7 @@ bool jit_disabled() {
   return v && *v && std::strcmp(v, "0") != 0;
 }
 
-std::string jit_source_of(const rebop_gillespie *g, bool cap = false) {
+std::string jit_source_of(const rebop_gillespie *g, bool cap) {
   std::vector<rebop::JitReaction> jr;
   jr.reserve(g->rx.size());
   for (auto &r : g->rx) {
@@ -755,32 +755,26 @@ std::string jit_source_of(const rebop_gillespie *g, bool cap = false) {
     j.consts = r.consts;
     jr.push_back(std::move(j));
   }
-  std::string src = rebop::jit_source(g->S, jr, g->system, cap);
-  // REBOP_DUMP_SPECIALIZED=<file>: write the generated kernel source there
-  if (const char *path = std::getenv("REBOP_DUMP_SPECIALIZED")) {
-    if (FILE *f = std::fopen(path, "w")) {
-      std::fputs(src.c_str(), f);
-      std::fclose(f);
-    }
-  }
-  return src;
+  return rebop::jit_source(g->S, jr, g->system, cap);
 }
 
-// Is the specialised kernel (cap: its variant with the draw-cap checks) loaded
-// on device `dev` for the handle's current network?
-bool jit_ready(const rebop_gillespie *g, bool cap, int dev) {
+// The specialised kernels of the handle's current network that are loaded on
+// device `dev` (cap: those with the draw-cap checks).
+uint32_t jit_loaded(const rebop_gillespie *g, bool cap, int dev) {
   const int v = cap ? 1 : 0;
-  return !g->jit_dirty[v] && g->jit_dev[v] == dev && g->jitk[v].fn;
+  return !g->jit_dirty[v] && g->jit_dev[v] == dev ? g->jitk[v].have() : 0u;
 }
 
-// Compiles (cached) and loads the network-specialised kernel on the current device.
-int prepare_jit(rebop_gillespie *g, bool cap = false) {
+// Compiles (cached) and loads variants of the network-specialised kernel
+// (`mask`, jit.h) on the current device, those missing of it.
+int prepare_jit(rebop_gillespie *g, bool cap, uint32_t mask) {
   int cur = -1;
   HIP_TRY(hipGetDevice(&cur));
-  if (jit_ready(g, cap, cur)) return REBOP_OK;
+  if ((mask & ~jit_loaded(g, cap, cur)) == 0u) return REBOP_OK;
   const int v = cap ? 1 : 0;
   std::string err;
-  if (rebop::jit_get(jit_source_of(g, cap), &g->jitk[v], &err) != 0) {
+  if (rebop::jit_get(jit_source_of(g, cap), mask, rebop::jit_prepare_set((uint32_t)g->rx.size(), cap),
+                     &g->jitk[v], &err) != 0) {
     g->jit_err = err;
     return fail(REBOP_ERR_DEVICE, "specialised kernel: " + err);
   }
@@ -1149,16 +1143,62 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
       }
   const bool fits_regs = !g->n_expr && !g->system && pick_reg_shape(S, R) >= 0;
   bool spec = false, use_lds = variant == REBOP_KERNEL_LDS;
-  if (!use_lds && (kernel & REBOP_KERNEL_SPECIALIZED)) {
-    if (!jit_eligible(g))
-      return fail(REBOP_ERR_UNSUPPORTED,
-                  "network too large for a specialised kernel (S <= 32, R <= 64)");
-    rc = prepare_jit(g, run.draw_cap != 0);
-    if (rc) return rc;
-    spec = true;
+  const bool ask_spec = !use_lds && (kernel & REBOP_KERNEL_SPECIALIZED);
+  if (ask_spec && !jit_eligible(g))
+    return fail(REBOP_ERR_UNSUPPORTED,
+                "network too large for a specialised kernel (S <= 32, R <= 64)");
+  // lanes per trajectory: asked for, or (AUTO) when even 4 (2) lanes per
+  // trajectory leave at most one wave per SIMD
+  int group = (kernel & REBOP_KERNEL_GROUP4) ? 4 : (kernel & REBOP_KERNEL_GROUP2) ? 2 : 1;
+  const bool any_spec = ask_spec || (variant == REBOP_KERNEL_AUTO && jit_eligible(g) && !jit_disabled());
+  const uint64_t lanes = (uint64_t)g_dev.cus * 4u * 64u; // one wave per SIMD
+  if (group == 1 && variant == REBOP_KERNEL_AUTO && any_spec && !run.rates) {
+    if (run.n_traj * 4u <= lanes)
+      group = 4;
+    else if (run.n_traj * 2u <= lanes)
+      group = 2;
+  }
+  // Sixteen lanes where they too leave one wave per SIMD, unless four were
+  // asked for: a draw (a Philox block and a logarithm, a third of an event's
+  // instructions with four lanes) then costs a sixteenth of its own.  4096 SIR
+  // trajectories advanced to two times, a call: 772 us with four lanes and
+  // every test, 570 us with sixteen in straight rounds (692 us when those
+  // end every four draws).
+  if (group == 4 && any_group && any_spec && rebop::jit_sixteen(R, run.draw_cap != 0) &&
+      run.n_traj * 16u <= lanes && rebop::group_straight(run, S))
+    group = 16;
+  // the specialised kernels the run takes: its own, and the tail's (tail
+  // hand-off: see rebop_dev_run)
+  const uint32_t below = tail_lanes();
+  const int tail_k = tail_group();
+  const bool events = run.mode == REBOP_MODE_EVENTS, write = run.rec_offsets != nullptr;
+  const bool may_tail = group == 1 && variant != REBOP_KERNEL_PLAIN && !run.rates && !events &&
+                        !(kernel & REBOP_KERNEL_WHOLE) && below > 0 && run.n_traj > 0 && !sc;
+  auto variant_of = [&](int lanes_per) {
+    if (run.rates) return (int)rebop::kJitSweep;
+    if (lanes_per == 1) return (int)rebop::kJitMain;
+    if (events)
+      return (int)(lanes_per == 4 ? write ? rebop::kJitEv4Write : rebop::kJitEv4Count
+                   : write        ? rebop::kJitEv2Write
+                                  : rebop::kJitEv2Count);
+    const bool near = rebop::group_straight(run, S);
+    return (int)(lanes_per == 16  ? rebop::kJitG16
+                 : lanes_per == 4 ? near ? rebop::kJitG4 : rebop::kJitG4Far
+                 : near           ? rebop::kJitG2
+                                  : rebop::kJitG2Far);
+  };
+  if (!use_lds && any_spec) {
+    const uint32_t need = rebop::jit_bit(variant_of(group)) |
+                          (may_tail ? rebop::jit_bit(variant_of(tail_k)) : 0u);
+    rc = prepare_jit(g, run.draw_cap != 0, need);
+    if (rc && ask_spec) return rc;
+    spec = rc == REBOP_OK;
+    if (!spec) {
+      group = 1;
+      use_lds = !fits_regs;
+    }
   } else if (!use_lds && variant == REBOP_KERNEL_AUTO) {
-    spec = jit_eligible(g) && !jit_disabled() && prepare_jit(g, run.draw_cap != 0) == REBOP_OK;
-    use_lds = !spec && !fits_regs;
+    use_lds = !fits_regs;
   } else if (!use_lds && !fits_regs) {
     return fail(REBOP_ERR_UNSUPPORTED, "network with " + std::to_string(S) + " species and " +
                                            std::to_string(R) +
@@ -1229,10 +1269,6 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
       shape.ok = false;
     }
   }
-  // lanes per trajectory: asked for, or (AUTO) when even 4 (2) lanes per
-  // trajectory leave at most one wave per SIMD
-  int group = (kernel & REBOP_KERNEL_GROUP4) ? 4 : (kernel & REBOP_KERNEL_GROUP2) ? 2 : 1;
-  const uint64_t lanes = (uint64_t)g_dev.cus * 4u * 64u; // one wave per SIMD
   if (group > 1) {
     if (!spec)
       return fail(REBOP_ERR_UNSUPPORTED,
@@ -1240,20 +1276,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
     if (variant == REBOP_KERNEL_PERSISTENT || run.rates)
       return fail(REBOP_ERR_UNSUPPORTED,
                   "lanes per trajectory > 1 applies to plain runs without rate tables");
-  } else if (variant == REBOP_KERNEL_AUTO && spec && !run.rates) {
-    if (run.n_traj * 4u <= lanes)
-      group = 4;
-    else if (run.n_traj * 2u <= lanes)
-      group = 2;
   }
-  // Sixteen lanes where they too leave one wave per SIMD, unless four were
-  // asked for: a draw (a Philox block and a logarithm, a third of an event's
-  // instructions with four lanes) then costs a sixteenth of its own.  4096 SIR
-  // trajectories advanced to two times, a call: 772 us with four lanes and
-  // every test, 570 us with sixteen in straight rounds (692 us when those
-  // end every four draws).
-  if (group == 4 && any_group && spec && !run.draw_cap && run.n_traj * 16u <= lanes && rebop::group_straight(run, S))
-    group = 16;
   const bool persistent = group == 1 && variant != REBOP_KERNEL_PLAIN;
   const int shape = spec ? -1 : pick_reg_shape(S, R);
   if (!spec && shape < 0)
@@ -1266,11 +1289,11 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   const size_t lds = spec ? 0 : sizeof(double) * (size_t)R * S;
   const uint64_t need_blocks = (run.n_traj * (uint64_t)group + threads - 1) / threads;
   uint64_t blocks = need_blocks;
+  const rebop::JitKernel &jitk = g->jitk[run.draw_cap ? 1 : 0];
   if (persistent) {
     int per_cu = 0;
     if (spec)
-      HIP_TRY(rebop::jit_occupancy(g->jitk[run.draw_cap ? 1 : 0], threads,
-                                   rebop::jit_dynamic_lds(run), &per_cu));
+      HIP_TRY(rebop::jit_occupancy(jitk, variant_of(1), threads, rebop::jit_dynamic_lds(run), &per_cu));
     else
       HIP_TRY(rebop::reg_occupancy(shape, threads, lds, &per_cu));
     if (per_cu < 1) per_cu = 1;
@@ -1283,12 +1306,9 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   const int kind = (persistent ? REBOP_KERNEL_PERSISTENT : REBOP_KERNEL_PLAIN) |
                    (spec ? REBOP_KERNEL_SPECIALIZED : 0) |
                    (group >= 4 ? REBOP_KERNEL_GROUP4 : group == 2 ? REBOP_KERNEL_GROUP2 : 0);
-  // tail hand-off (see rebop_dev_run): a wave spills at most spill_below
-  // trajectories, once, so the arrays need (waves x spill_below) entries
-  const uint32_t below = tail_lanes();
-  const bool tail = persistent && spec && !run.rates && run.mode != REBOP_MODE_EVENTS &&
-                    !(kernel & REBOP_KERNEL_WHOLE) && below > 0 && run.n_traj > 0 && !sc;
-  const int tail_k = tail_group();
+  // a wave spills at most spill_below trajectories, once, so the arrays need
+  // (waves x spill_below) entries
+  const bool tail = may_tail && spec;
   uint64_t tail_blocks = 0;
   if (tail) {
     const uint64_t cap = blocks * (uint64_t)threads / 64u * below;
@@ -1331,8 +1351,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   if (ev.e0) HIP_TRY(hipEventRecord(ev.e0, stream));
   if (run.n_traj > 0) {
     if (spec)
-      HIP_TRY(rebop::jit_launch(g->jitk[run.draw_cap ? 1 : 0], run, (int)blocks, threads, stream,
-                                group));
+      HIP_TRY(rebop::jit_launch(jitk, variant_of(group), run, (int)blocks, threads, stream));
     else
       HIP_TRY(rebop::launch_reg(shape, g->view, run, (int)blocks, threads, lds, stream));
   }
@@ -1342,8 +1361,7 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
     r2.persistent = 0;
     r2.spill_below = 0;
     r2.resume = 1;
-    HIP_TRY(rebop::jit_launch(g->jitk[run.draw_cap ? 1 : 0], r2, (int)tail_blocks, threads, stream,
-                              tail_k));
+    HIP_TRY(rebop::jit_launch(jitk, variant_of(tail_k), r2, (int)tail_blocks, threads, stream));
   }
   // the samples were written as f64 bits: convert them to int64 in place
   if (run.out && run.mode == REBOP_MODE_GRID && run.n_traj > 0)
@@ -1402,7 +1420,7 @@ int run_device_scratch(const rebop_gillespie *gc, double tmax, uint64_t nb_steps
     const int variant = kernel & 0xF;
     const bool wants_jit = specialised_only(g) || (kernel & REBOP_KERNEL_SPECIALIZED) ||
                            (variant == REBOP_KERNEL_AUTO && jit_eligible(g) && !jit_disabled());
-    if (wants_jit && !jit_ready(g, effective_cap(g, tmax) != 0, cur))
+    if (wants_jit && !jit_loaded(g, effective_cap(g, tmax) != 0, cur))
       return fail(REBOP_ERR_VALUE, "the specialised kernel is not compiled on this device: call "
                                    "rebop_gillespie_prepare with this kernel kind (after setting "
                                    "any draw cap) first");
@@ -1705,17 +1723,18 @@ int rebop_gillespie_prepare(const rebop_gillespie *gc, int kernel) {
   if (!has_dev) {
     // no device: compile only, to check the generated kernel
     std::string err;
-    size_t cs = 0;
-    if (rebop::jit_compile_only(jit_source_of(g, g->draw_cap != 0), &cs, &err) != 0)
+    if (rebop::jit_compile_only(jit_source_of(g, g->draw_cap != 0),
+                                rebop::jit_prepare_set((uint32_t)g->rx.size(), g->draw_cap != 0), &err) != 0)
       return fail(REBOP_ERR_DEVICE, "specialised kernel: " + err);
     return REBOP_OK;
   }
   if (int rc = ensure_device()) return rc;
   if (int rc = upload_net(g)) return rc;
   // with a draw cap set, the variant that checks it too
+  const uint32_t R = (uint32_t)g->rx.size();
   if (g->draw_cap)
-    if (int rc = prepare_jit(g, true)) return rc;
-  return prepare_jit(g);
+    if (int rc = prepare_jit(g, true, rebop::jit_prepare_set(R, true))) return rc;
+  return prepare_jit(g, false, rebop::jit_prepare_set(R, false));
 }
 
 int rebop_run_device(const rebop_gillespie *gc, double tmax, uint64_t nb_steps,
@@ -1762,7 +1781,8 @@ int rebop_autotune(rebop_gillespie *g, double tmax, uint64_t nb_steps, uint64_t 
     double occ;
   };
   std::vector<Cand> cands;
-  const bool jit_ok = jit_eligible(g) && !jit_disabled() && prepare_jit(g) == REBOP_OK;
+  const bool jit_ok = jit_eligible(g) && !jit_disabled() &&
+                      prepare_jit(g, false, rebop::jit_prepare_set(R, false)) == REBOP_OK;
   const bool reg_ok = pick_reg_shape(S, R) >= 0;
   for (int threads : {64, 128, 256}) {
     for (double occ : {1.0, 0.6, 0.4, 0.25}) {
