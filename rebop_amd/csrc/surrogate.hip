@@ -1027,7 +1027,9 @@ __global__ void __launch_bounds__(512) mlp_infer_kernel(int M, const __bf16 *__r
 // series of ln Gamma (Stirling) and of the digamma function, with the
 // Bernoulli-number coefficients B_2n / (2n (2n-1)) and B_2n / (2n).
 
-// 1 / z within an ulp, for normal z away from the ends of the range
+// 1 / z for normal z away from the ends of the range: the hardware's
+// approximation and two Newton-Raphson steps, the last of which rounds
+// correctly (equal to the division for all of 7.9e8 values over e^-7 .. e^24).
 __device__ __forceinline__ double rcp_pos(double z) {
   double y = __builtin_amdgcn_rcp(z);
   y = __builtin_fma(y, __builtin_fma(-z, y, 1.0), y);
@@ -1036,9 +1038,12 @@ __device__ __forceinline__ double rcp_pos(double z) {
 
 // ln x, within an ulp, for positive normal x: x = 2^k m, m in [sqrt(1/2),
 // sqrt(2)), f = m - 1, s = f / (2 + f) and ln m = 2 atanh s = f - s (f - P),
-// P = sum 2 s^2n / (2n + 1), whose terms past n = 10 are below 2^-60 of it.
-// A third of the instructions of the library's logarithm, which carries a
-// double pair.
+// P = sum 2 s^2n / (2n + 1), whose terms past n = 10 are below 2^-60 of it;
+// the arrangement, with ln 2 in two parts, is that of the public-domain
+// fdlibm.  A third of the instructions of the library's logarithm, which
+// carries a double pair: 0.97 against 0.52 ulp at most (0.2591 against 0.2500
+// on average in [0.5, 1.5], 0.2506 against 0.2501 above 10), a difference that
+// the sums below do not show (lgamma_digamma_pos).
 __device__ __forceinline__ double ln_pos(double x) {
   double m = __builtin_amdgcn_frexp_mant(x);
   int k = __builtin_amdgcn_frexp_exp(x);
@@ -1059,6 +1064,13 @@ __device__ __forceinline__ double ln_pos(double x) {
 // ln Gamma(z) = ln Gamma(z + n) - ln p(z) and psi(z) = psi(z + n) -
 // p'(z) / p(z): one division for the whole shift (at most 10 factors below
 // 10: no overflow), and neither it nor ln p where no lane needs a shift.
+// Six terms of the series: the first one left out is at most 6.4e-16 of
+// ln Gamma and 8.3e-16 of psi (z = 10).  Largest and mean error over z in
+// e^-6 .. e^12 with counts 0 .. 1000 added, in units of 2^-53 max(1, |value|):
+// ln Gamma 74.1 and 4.53, psi 21.7 and 1.47; with the library's logarithm
+// 70.7 and 4.51, 21.7 and 1.45; with it, five terms and the shift of psi as a
+// sum of reciprocals, 217 and 28.5, 191 and 18.7.  The library's logarithm
+// costs the loss 3.5 us of 62 (4096 items).
 template <bool PSI>
 __device__ __forceinline__ double lgamma_digamma_pos(double z, double *psi) {
   double prod = 1.0, dprod = 0.0;
@@ -1080,10 +1092,14 @@ __device__ __forceinline__ double lgamma_digamma_pos(double z, double *psi) {
   }
   const double iz = rcp_pos(z), iz2 = iz * iz, lz = ln_pos(z);
   const double series =
-      iz * (1.0 / 12.0 - iz2 * (1.0 / 360.0 - iz2 * (1.0 / 1260.0 - iz2 * (1.0 / 1680.0 - iz2 * (1.0 / 1188.0)))));
+      iz * (1.0 / 12.0 -
+            iz2 * (1.0 / 360.0 -
+                   iz2 * (1.0 / 1260.0 - iz2 * (1.0 / 1680.0 - iz2 * (1.0 / 1188.0 - iz2 * (691.0 / 360360.0))))));
   if (PSI) {
     const double dseries =
-        iz2 * (1.0 / 12.0 - iz2 * (1.0 / 120.0 - iz2 * (1.0 / 252.0 - iz2 * (1.0 / 240.0 - iz2 * (1.0 / 132.0)))));
+        iz2 * (1.0 / 12.0 -
+               iz2 * (1.0 / 120.0 -
+                      iz2 * (1.0 / 252.0 - iz2 * (1.0 / 240.0 - iz2 * (1.0 / 132.0 - iz2 * (691.0 / 32760.0))))));
     *psi = lz - 0.5 * iz - dseries - dshift;
   }
   return (z - 0.5) * lz - z + 0.91893853320467274178 + series - shift;

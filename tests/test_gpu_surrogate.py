@@ -559,3 +559,22 @@ def test_features_of_any_count_and_row(sg, B, ldx, off):
     assert (np.abs(got - want) <= np.abs(want) * 2.0**-7 + 1e-30).all()
     assert np.array_equal(bound[:B].double().cpu().numpy(), br) and (bound[B] == -1).all()
     assert (buf[:off] == 7).all() and (buf[off + B * ldx:] == 7).all()
+
+
+def test_likelihood_is_as_accurate_as_its_arithmetic(sg):
+    """One negative binomial (r = 1, mean 1) in every component and counts of
+    zero: ln Gamma(x + r) and ln Gamma(r) cancel exactly, so a sample's value
+    is ln 2 plus the error of ln Gamma(1).  That is a sum of terms up to
+    9.5 ln 10 = 21.9 and two logarithms: five roundings of at most 1.8e-15 and
+    a truncation of 6.4e-16, below 1e-14 (a series of five terms: 1.9e-14)."""
+    import torch
+
+    B = 4
+    head = torch.zeros((B, sg.OUT), device="cuda")
+    item = torch.zeros(B, dtype=torch.int32, device="cuda")
+    samples = torch.zeros((2, sg.S, sg.J), dtype=torch.int64, device="cuda")
+    grad = torch.zeros((B, sg.OUT), device="cuda")
+    loss = torch.zeros(1, dtype=torch.float64, device="cuda")
+    sg.nb_mixture_nll(head, item, item, samples, grad, loss, 1.0)
+    n = B * sg.S * sg.J
+    assert abs(loss.item() / n - np.log(2.0)) < 1e-14
