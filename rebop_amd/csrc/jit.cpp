@@ -121,7 +121,7 @@ std::string jit_source(uint32_t S, const std::vector<JitReaction> &rx, bool syst
   s += "  __device__ __forceinline__ void store_state(const X &x, double *st, uint64_t stride) const { rebop::reg_store_state(x, st, stride, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ void write_counts(const X &x, int64_t *dst, uint64_t stride) const { rebop::reg_write_counts(x, dst, stride, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ void write_raw(const X &x, int64_t *dst, uint64_t stride) const { rebop::reg_write_raw(x, dst, stride, " + Ss + "); }\n";
-  s += "  __device__ __forceinline__ void write_raw_buffer(const X &x, rebop::WordBuffer b, uint32_t at, uint32_t stride) const { rebop::reg_write_raw_buffer(x, b, at, stride, " + Ss + "); }\n";
+  s += "  __device__ __forceinline__ void write_raw_buffer(const X &x, rebop::ByteBuffer b, uint32_t at, uint32_t stride) const { rebop::reg_write_raw_buffer(x, b, at, stride, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ bool small(const X &x) const { return rebop::reg_small(x, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ void write_small(const X &x, int64_t *dst) const { rebop::reg_write_small(x, dst, " + Ss + "); }\n";
   s += "  __device__ __forceinline__ bool in_range(const X &x) const { return rebop::reg_in_range(x, " + Ss + "); }\n";

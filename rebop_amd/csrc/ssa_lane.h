@@ -128,30 +128,29 @@ __device__ __forceinline__ void reg_write_raw(const double (&x)[MS], int64_t *ds
     if (s < (int)S) dst[(uint64_t)s * stride] = (int64_t)rebop_f64_bits(x[s]);
 }
 
-// A buffer of `n` 8-byte words at p (below 2^31 of them): stores at a word's
-// index, dropped where it is past the end.
+// A buffer of `n` bytes at p (below 4 GiB): stores at a byte offset, dropped
+// where that is n or more.
 #if defined(__HIP_DEVICE_COMPILE__)
-typedef __amdgpu_buffer_rsrc_t WordBuffer;
+typedef __amdgpu_buffer_rsrc_t ByteBuffer;
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-__device__ void word_buffer_store(u32x2_t v, WordBuffer buf, int index, int offset, int soffset,
-                                  int aux) __asm("llvm.amdgcn.struct.ptr.buffer.store.v2i32");
-__device__ __forceinline__ WordBuffer word_buffer(void *p, uint32_t n) {
-  return __builtin_amdgcn_make_buffer_rsrc(p, 8, (int)n, 0x00020000);
+__device__ __forceinline__ ByteBuffer byte_buffer(void *p, uint32_t n) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, 0, (int)n, 0x00020000);
 }
 #else
-struct WordBuffer {};
-__device__ __forceinline__ WordBuffer word_buffer(void *, uint32_t) { return WordBuffer{}; }
+struct ByteBuffer {};
+__device__ __forceinline__ ByteBuffer byte_buffer(void *, uint32_t) { return ByteBuffer{}; }
 #endif
-// reg_write_raw to word `at`, the species `stride` words apart
+// reg_write_raw to byte `at`, the species `stride` bytes apart
 template <int MS>
-__device__ __forceinline__ void reg_write_raw_buffer(const double (&x)[MS], WordBuffer buf, uint32_t at,
+__device__ __forceinline__ void reg_write_raw_buffer(const double (&x)[MS], ByteBuffer buf, uint32_t at,
                                                      uint32_t stride, uint32_t S) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
   for (int s = 0; s < MS; ++s)
     if (s < (int)S) {
       const uint64_t b = rebop_f64_bits(x[s]);
-      word_buffer_store(u32x2_t{(uint32_t)b, (uint32_t)(b >> 32)}, buf, (int)at, 0, (int)(s * stride * 8u), 0);
+      __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{(uint32_t)b, (uint32_t)(b >> 32)}, buf, (int)at,
+                                            (int)(s * stride), 0);
     }
 #endif
 }
@@ -542,7 +541,7 @@ __device__ __forceinline__ void group_steps(F &&f) {
 // way: until it is absorbed, a trajectory takes a draw in every iteration and
 // overshoots once per sample.  The range of the counts is checked once a round.
 //
-// Straight rounds (sample times in LDS, an output below 2^31 counts or none, no
+// Straight rounds (sample times in LDS, an output below 4 GiB or none, no
 // draw cap) have no branch at all.  Samples are stored with buffer instructions whose
 // bounds check drops the lanes that have none.  A trajectory past its last
 // sample time reads NaN for the next, so it keeps recording, out of bounds,
@@ -664,11 +663,13 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
       acc.trajectories += 1;
     }
   };
-  // the straight rounds' stores: 32-bit indices into run.out, and a lane that
-  // writes nothing has one that the buffer's bounds check drops
-  constexpr uint32_t kDrop = 0x80000000u;
-  const uint32_t row = (uint32_t)Sn;
-  const WordBuffer out = word_buffer(run.out, FAST && run.out ? (nb + 1u) * row : 0u);
+  // the straight rounds' stores: 32-bit byte offsets into run.out, and a lane
+  // that writes nothing stores past its end (by a round's samples at most, so
+  // below 4 GiB: group_straight), where the buffer's bounds check drops it.
+  // Without run.out the buffer is empty and every offset zero.
+  const uint32_t row = FAST && run.out ? (uint32_t)Sn * 8u : 0u;
+  const uint32_t stride = FAST && run.out ? (uint32_t)n * 8u : 0u, past = (nb + 1u) * row;
+  const ByteBuffer out = byte_buffer(run.out, past);
 
   // this lane's draw of the next round: ln reduced and its table row read,
   // the rest of the ln evaluated when the round starts
@@ -689,7 +690,7 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
 #pragma unroll
       for (int s = 0; s < Net::MS; ++s) xs[s] = x[s];
       const uint32_t is = i;
-      uint32_t at = (lead ? 0u : kDrop) + i * row + (uint32_t)jl, worst = 0;
+      uint32_t at = lead ? i * row + (run.out ? (uint32_t)jl * 8u : 0u) : past, worst = 0;
       fetch(d0 + K);
       group_steps<K>([&](auto step) {
         constexpr int q = decltype(step)::q;
@@ -705,20 +706,20 @@ __device__ __forceinline__ LaneTotals lane_loop_group(Net &net, const rebop_dev_
         const uint32_t far = usual_distance(total);
         const uint32_t seen = rec ? 0u : far;
         worst = worst > seen ? worst : seen;
-        net.write_raw_buffer(x, out, rec ? at : kDrop, (uint32_t)n);
+        net.write_raw_buffer(x, out, rec ? at : past, stride);
         at += rec ? row : 0u;
         T = rec ? Tn : T;
         i += rec ? 1u : 0u;
         Tn = grid_lds[i + 1u];
       });
       if (__builtin_expect(__ballot(worst >= kUsualSpan) == 0ull, 1)) {
-        const uint32_t past = i > nb ? i - nb - 1u : 0u; // samples past the last one
-        i -= past;
+        const uint32_t extra = i > nb ? i - nb - 1u : 0u; // samples past the last one
+        i -= extra;
         const bool last = i > nb && !finished;
         if (__builtin_expect(__ballot(last) != 0ull, 0))
           if (last) {
             t = grid_lds[nb];
-            finish(d0 + (K - past));
+            finish(d0 + (K - extra));
           }
         draw = d0 + K;
         continue;

@@ -143,16 +143,15 @@ inline uint64_t run_samples(const rebop_dev_run &run) {
   return run.mode == REBOP_MODE_TARGET ? 1u : run.nb_steps + 1u;
 }
 /* Whether a grouped launch over S species may take straight rounds: the sample
- * times fit LDS, and the stores' 32-bit indices, which run a round past the
- * output, stay below 2^31 (and a sample's counts below 2^32 bytes). */
+ * times fit LDS, and the stores' 32-bit byte offsets, which run a round past
+ * the output, stay below 2^32. */
 #if defined(__HIPCC__) || defined(__HIPCC_RTC__)
 __host__ __device__
 #endif
 inline bool group_straight(const rebop_dev_run &run, uint32_t S) {
   const uint64_t n = run_samples(run);
   return run.mode != REBOP_MODE_EVENTS && n <= REBOP_GRID_LDS &&
-         (!run.out || ((n + REBOP_GRID_PAD) * run.n_traj < 0x80000000ull / (S ? S : 1u) &&
-                       run.n_traj < 0x20000000ull / (S ? S : 1u)));
+         (!run.out || run.n_traj < 0x20000000ull / ((n + REBOP_GRID_PAD) * (S ? S : 1u)));
 }
 } // namespace rebop
 #endif
