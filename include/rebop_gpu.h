@@ -71,7 +71,7 @@ enum rebop_kernel_kind {
                                   reaction must fit one workgroup's LDS (160 KB).  Also
                                   reported where AUTO or a job batch ran the incremental
                                   kernel (eight lanes per trajectory, counts in LDS), whose
-                                  results are the same */
+                                  results are the same (rebop_last_kernel tells them apart) */
   /* flag: the network compiled into the kernel (run-time compilation,
    * cached); combine with PLAIN or PERSISTENT */
   REBOP_KERNEL_SPECIALIZED = 16,
@@ -430,6 +430,22 @@ int rebop_batch_set_draws(rebop_batch *b, const uint64_t *draws);
 
 /* Description of the last error on this thread ("" if none). */
 const char *rebop_last_error(void);
+
+/* The kernel that the calling thread's last run launched, where
+ * rebop_stats.kernel has one value for several (valid until the thread's next
+ * run; "" before the first):
+ *   "lds:int16", "lds:int32", "lds:int64"  the LDS kernel, by its counts
+ *   "incremental", "incremental:stored", "incremental:expr"  the incremental
+ *       kernel: propensities evaluated again or kept in LDS, or a network with
+ *       rate expressions
+ *   "register:plain", "register:persistent"  the data-driven register kernels
+ *   "specialized:<form>"  a specialised kernel: main (one lane per
+ *       trajectory), g2, g4, g16 (that many lanes), g2_far and g4_far (the
+ *       sample times computed, or an output past 4 GiB: step-by-step rounds),
+ *       sweep (rate tables), ev2_count, ev2_write, ev4_count and ev4_write
+ *       (every event recorded with 2 or 4 lanes); "+g4" after it is the tail
+ * "a > b": the launch of a was replaced by one of b, whose counts are wider. */
+const char *rebop_last_kernel(void);
 
 /* Name of the device the library runs on, and its compute-unit count. */
 int rebop_device_info(char *name, size_t name_len, int *cu_count);

@@ -123,6 +123,7 @@ SIGNATURES: dict[str, tuple] = {
          POINTER(c_uint32), POINTER(c_uint32), c_uint32],
     ),
     "rebop_last_error": (c_char_p, []),
+    "rebop_last_kernel": (c_char_p, []),
     "rebop_device_info": (c_int, [c_char_p, c_size_t, POINTER(c_int)]),
 }
 
@@ -226,6 +227,11 @@ def check(code: int) -> None:
     if code == REBOP_ERR_CAP:
         raise RebopCapError(code, msg)
     raise RebopError(code, msg)
+
+
+def last_kernel() -> str:
+    """The kernel that this thread's last run took (``rebop_last_kernel``)."""
+    return load().rebop_last_kernel().decode()
 
 
 def device_info() -> tuple[str, int]:

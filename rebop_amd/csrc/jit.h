@@ -46,6 +46,7 @@ enum JitVariant {
   kJitVariants
 };
 constexpr uint32_t jit_bit(int variant) { return 1u << variant; }
+const char *jit_variant_name(int variant);
 
 struct JitKernel {
   hipFunction_t fn[kJitVariants] = {};

@@ -60,6 +60,13 @@ hipError_t launch_inc(const rebop_dev_job *jobs, const uint32_t *tickets, uint32
 namespace {
 
 thread_local std::string g_last_error;
+thread_local std::string g_last_kernel;
+
+// What rebop_last_kernel reports: the kernel of a launch, or (`again`) that of
+// the launch that replaces the one named before.
+void note_kernel(const std::string &name, bool again) {
+  g_last_kernel = again ? g_last_kernel + " > " + name : name;
+}
 
 int fail(int code, const std::string &msg) {
   g_last_error = msg;
@@ -851,6 +858,8 @@ int lds_kind(int width) {
   return REBOP_KERNEL_LDS | (width == 8 ? REBOP_KERNEL_WIDE : width == 2 ? REBOP_KERNEL_COMPACT : 0);
 }
 
+std::string lds_name(int width) { return "lds:int" + std::to_string(8 * width); }
+
 // The LDS of one workgroup of an LDS launch: counts [1 + S_max][64] of
 // `width` bytes (row 0 holds ones, for absent factors; 16-byte aligned),
 // then the reaction records and four of padding, unless they are read in
@@ -1012,6 +1021,10 @@ IncShape inc_shape(const std::vector<rebop_dev_job> &jobs, bool store, uint32_t 
   }
   s.ok = s.per_cu > 0 && (s.expr || inc_pays(jobs));
   return s;
+}
+
+std::string inc_name(const IncShape &s) {
+  return s.expr ? "incremental:expr" : s.store ? "incremental:stored" : "incremental";
 }
 
 // Uploads the job and ticket tables and enqueues the incremental kernel.
@@ -1247,9 +1260,10 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
     IncShape shape;
     if (any_lds && !sc && width < 8)
       shape = inc_shape(std::vector<rebop_dev_job>{job}, g->inc_store, g->inc_depth);
-    for (;;) {
+    for (bool again = false;; again = true) {
       EventPair ev;
       if (stats && !sc) HIP_TRY(ev.create());
+      note_kernel(shape.ok ? inc_name(shape) : lds_name(width), again);
       HIP_TRY(rebop::launch_reset_counters(ctrs, stream));
       if (ev.e0) HIP_TRY(hipEventRecord(ev.e0, stream));
       if (shape.ok)
@@ -1330,6 +1344,10 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
     tail_blocks = (cap * (uint64_t)tail_k + threads - 1) / threads;
   }
 
+  note_kernel(spec ? std::string("specialized:") + rebop::jit_variant_name(variant_of(group)) +
+                         (tail ? std::string("+") + rebop::jit_variant_name(variant_of(tail_k)) : "")
+                   : persistent ? "register:persistent" : "register:plain",
+              false);
   EventPair ev;
   if (stats && !sc) HIP_TRY(ev.create());
   HIP_TRY(rebop::launch_reset_counters(run.counters, stream));
@@ -1380,7 +1398,10 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
       return fail(REBOP_ERR_RANGE, std::string("a count left the exactly simulated range |x| <= "
                                                "2^52 of ") +
                                        (run.rates ? "a run with rate tables" : "a resumable batch"));
-    return launch_run(g, run_in, REBOP_KERNEL_LDS | REBOP_KERNEL_WIDE, stream, stats, 0, 1.0, sc);
+    const std::string first = g_last_kernel;
+    rc = launch_run(g, run_in, REBOP_KERNEL_LDS | REBOP_KERNEL_WIDE, stream, stats, 0, 1.0, sc);
+    g_last_kernel = first + " > " + g_last_kernel;
+    return rc;
   }
   return REBOP_OK;
 }
@@ -1447,6 +1468,7 @@ int run_device_scratch(const rebop_gillespie *gc, double tmax, uint64_t nb_steps
 extern "C" {
 
 const char *rebop_last_error(void) { return g_last_error.c_str(); }
+const char *rebop_last_kernel(void) { return g_last_kernel.c_str(); }
 
 int rebop_device_info(char *name, size_t name_len, int *cu_count) {
   int rc = ensure_device();
@@ -1986,7 +2008,8 @@ int rebop_run_jobs_device(const rebop_job *jobs, uint32_t n_jobs, void *stream_,
     shape = inc_shape(dj, store, depth);
   }
   rebop_stats local{};
-  for (;;) {
+  for (bool again = false;; again = true) {
+    note_kernel(shape.ok ? inc_name(shape) : lds_name(width), again);
     if (jev) HIP_TRY(rebop::launch_zero_u64(jev, n_jobs, stream));
     HIP_TRY(rebop::launch_zero_u64(jq, n_jobs, stream));
     EventPair ev;
