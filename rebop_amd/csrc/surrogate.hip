@@ -18,7 +18,6 @@
 #include <stdint.h>
 
 #include <type_traits>
-#include <vector>
 
 #include "../../include/rebop_surrogate.h"
 
@@ -1532,15 +1531,14 @@ int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead,
   hipStream_t s = (hipStream_t)stream;
   float *part = (float *)workspace, *colsum = part + p.part;
   __bf16 *dz = (__bf16 *)(colsum + p.colsum); // p.part and p.colsum are multiples of 64
-  size_t dz_end = p.dz;
+  // dZ from the last layer to the first, each with its column sums; a layer's
+  // dZ lies behind those of the layers before it
   int col = p.nbias;
-  auto layer_dz = [&](int l) { return dz + dz_end - (size_t)B * dims[l + 1]; };
-  // dZ from the last layer to the first, each with its column sums
-  std::vector<const __bf16 *> dZ((size_t)depth);
+  const __bf16 *next = nullptr; // dZ of layer l + 1
   for (int l = depth - 1; l >= 0; --l) {
     const int n = dims[l + 1];
-    __bf16 *out = layer_dz(l);
     col -= n;
+    __bf16 *out = dz + (size_t)B * col;
     if (l == depth - 1) {
       hipLaunchKernelGGL(sg::head_grad_kernel, dim3(n / 64, B / 64), dim3(256), 0, s, n, dhead, ldd, out,
                          colsum + col, p.nbias);
@@ -1553,15 +1551,15 @@ int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead,
       e.ldc = p.nbias;
       const bool big = big_tiles(B, n);
       const int tile = big ? 128 : 64, k = dims[l + 2];
-      launch_nt<sg::EPI_MASK>(big, dim3(n / tile, B / tile), s, B, n, k, dZ[l + 1], k, (const __bf16 *)Wb[l + 1], k,
+      launch_nt<sg::EPI_MASK>(big, dim3(n / tile, B / tile), s, B, n, k, next, k, (const __bf16 *)Wb[l + 1], k,
                               nullptr, 0, e);
     }
-    dZ[l] = out;
-    dz_end -= (size_t)B * n;
+    next = out;
   }
   // every layer's weight gradient
   float *wout = p.splits > 1 ? part : grads;
   size_t at = 0;
+  col = 0;
   for (int l0 = 0; l0 < depth; l0 += sg::WG_MAXL) {
     sg::WgradNet net{};
     int tiles = 0;
@@ -1569,13 +1567,14 @@ int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead,
       const int i = l - l0;
       net.H[i] = (const __bf16 *)(l == 0 ? X : H[l - 1]);
       net.ldh[i] = l == 0 ? ldx : dims[l];
-      net.dZ[i] = dZ[l];
+      net.dZ[i] = dz + (size_t)B * col;
       net.n[i] = dims[l + 1];
       net.tile0[i] = tiles;
       net.out[i] = at;
       net.layers = i + 1;
       tiles += (dims[l] / 64) * (dims[l + 1] / 64);
       at += (size_t)dims[l] * dims[l + 1];
+      col += dims[l + 1];
     }
     hipLaunchKernelGGL(sg::wgrad_kernel, dim3(tiles * p.splits), dim3(256), 0, s, p.units, p.splits, net, wout,
                        p.weights);
