@@ -53,7 +53,9 @@ int rebop_sg_gemm_bias_act_bf16(int tb, int M, int N, int K, const void *A, int 
  * bias[l]; H[l] (l < depth - 1) receives the hidden activations
  * [B][dims[l+1]] (BF16, after ReLU) and head the last layer's FP32 result
  * [B][dims[depth]].  The values of rebop_sg_gemm_bias_act_bf16 layer by layer.
- * B and all widths multiples of 64.  dims, Wt, bias and H are host arrays. */
+ * B and all widths multiples of 64, ldx a multiple of 8.  dims, Wt, bias and H
+ * are host arrays; no pointer needs more than its element's alignment (rows
+ * that start on 16 bytes are read and written fastest). */
 int rebop_sg_mlp_train_forward(int B, const void *X, int ldx, int depth, const int *dims,
                                const void *const *Wt, const float *const *bias, void *const *H,
                                float *head, void *stream);
@@ -68,8 +70,9 @@ size_t rebop_sg_mlp_backward_workspace(int B, int depth, const int *dims);
  * every layer's bias gradient (FP32).  Gradients between layers are FP32
  * until ReLU's derivative is applied, then BF16; bias gradients are summed
  * from the FP32 values.  Sums are taken in a fixed order: the same inputs
- * give the same bits.  H, Wb, workspace and grads 16-byte aligned, ldx a
- * multiple of 8, B and all widths multiples of 64. */
+ * give the same bits.  H, Wb, workspace and grads 16-byte aligned (3 if not),
+ * X and dhead aligned to their elements, ldx a multiple of 8, B and all widths
+ * multiples of 64. */
 int rebop_sg_mlp_backward(int B, int depth, const int *dims, const float *dhead, int ldd,
                           const void *X, int ldx, const void *const *H, const void *const *Wb,
                           void *workspace, float *grads, void *stream);

@@ -578,3 +578,60 @@ def test_likelihood_is_as_accurate_as_its_arithmetic(sg):
     sg.nb_mixture_nll(head, item, item, samples, grad, loss, 1.0)
     n = B * sg.S * sg.J
     assert abs(loss.item() / n - np.log(2.0)) < 1e-14
+
+
+@pytest.mark.parametrize("B,width,depth", [(64, 64, 1), (64, 128, 2), (320, 256, 4), (4096, 512, 5)])
+def test_training_passes_against_a_launch_per_step(sg, B, width, depth):
+    """The backward pass as products, ReLU derivative, BF16 casts and column
+    sums of their own: the same dZ bit for bit, so the gradients differ only
+    by the order of FP32 additions, each sum of B terms by at most 2 B 2^-24 of
+    the sum of their magnitudes."""
+    import torch
+
+    mlp = sg.MLP(seed=B + depth, width=width, depth=depth)
+    gen = torch.Generator(device="cuda").manual_seed(B)
+    X = torch.randn((B, sg.IN), generator=gen, device="cuda").to(torch.bfloat16)
+    dhead = torch.randn((B, sg.OUT), generator=gen, device="cuda")
+    mlp.forward(X)
+    H = list(mlp._H)
+    dW, db = mlp.backward(dhead)
+    dH = dhead.clone()
+    tol = 2.0 * B * 2.0**-24
+    for l in reversed(range(depth)):
+        dZ = torch.empty(dH.shape, dtype=torch.bfloat16, device="cuda")
+        if l == depth - 1:
+            sg.cast_bf16(dH, dZ)
+        else:
+            sg.relu_grad(dH, H[l + 1], dZ)  # dH too
+        b = torch.empty(dH.shape[1], device="cuda")
+        sg.colsum(dH, b)
+        assert bool(((db[l] - b).abs().double() <= tol * dH.double().abs().sum(0)).all()), l
+        w = torch.zeros(dW[l].shape, device="cuda")
+        sg.gemm(H[l], dZ, w, ta=True)
+        mag = H[l].double().abs().t() @ dZ.double().abs()
+        assert bool(((dW[l] - w).abs().double() <= tol * mag).all()), l
+        if l > 0:
+            dH = torch.empty((B, mlp.dims[l]), device="cuda")
+            sg.gemm(dZ, mlp.Wb[l], dH, tb=True)
+
+
+def test_training_passes_on_inputs_off_16_bytes(sg):
+    """X and dhead need only their elements' alignment."""
+    import torch
+
+    mlp = sg.MLP(seed=2, width=128, depth=3)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    X = torch.randn((64, sg.IN), generator=gen, device="cuda").to(torch.bfloat16)
+    dhead = torch.randn((64, sg.OUT), generator=gen, device="cuda")
+    head = mlp.forward(X)
+    dW, db = mlp.backward(dhead)
+    xb = torch.zeros(X.numel() + 1, dtype=torch.bfloat16, device="cuda")
+    gb = torch.zeros(dhead.numel() + 1, device="cuda")
+    x, g = xb[1:].view(X.shape), gb[1:].view(dhead.shape)
+    x.copy_(X)
+    g.copy_(dhead)
+    head2 = mlp.forward(x)
+    dW2, db2 = mlp.backward(g)
+    assert torch.equal(head, head2)
+    for a, b in zip(dW + db, dW2 + db2):
+        assert torch.equal(a, b)
