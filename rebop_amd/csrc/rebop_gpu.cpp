@@ -1174,9 +1174,9 @@ int launch_run(rebop_gillespie *g, rebop_dev_run run, int kernel, hipStream_t st
   // Sixteen lanes where they too leave one wave per SIMD, unless four were
   // asked for: a draw (a Philox block and a logarithm, a third of an event's
   // instructions with four lanes) then costs a sixteenth of its own.  4096 SIR
-  // trajectories advanced to two times, a call: 772 us with four lanes and
-  // every test, 570 us with sixteen in straight rounds (692 us when those
-  // end every four draws).
+  // trajectories advanced to two times, a call: 725 us with four lanes and
+  // branched rounds, 772 us with their one-path form and its tests, 575 us with
+  // sixteen lanes in straight rounds (692 us when those end every four draws).
   if (group == 4 && any_group && any_spec && rebop::jit_sixteen(R, run.draw_cap != 0) &&
       run.n_traj * 16u <= lanes && rebop::group_straight(run, S))
     group = 16;

@@ -46,18 +46,19 @@
 // block of the j-th of the next eight, which the group reads back from LDS one
 // per event), the changed reactions (lane j takes every eighth), the scans of
 // eight sums (three DPP steps) and the samples.  Counts (int32) and sums are
-// in LDS, about 9 KB a wave for 128 species and 512 reactions; the network's
+// in LDS, 10.3 KB a wave for 128 species and 512 reactions; the network's
 // tables (reaction records, jump records with the list of reactions each jump
 // changes) are read through the caches.
 //
-// What bounds it: VALU issue (68 % busy with 15 waves per CU on the 128 x 512
-// network, 38 wave instructions per event against 189 of the LDS kernel), and
-// for few trajectories the chain of dependent LDS reads, table reads and DPP
-// steps of an event.  Measured against the LDS kernel: 128 species x 512
+// What bounds it: VALU issue (69 % of the CU cycles with 15 waves per CU on the
+// 128 x 512 network, 39 wave instructions per event against 189 of the LDS
+// kernel) and the latency of an event's dependent table and LDS reads (the
+// waves wait on a counter half of their time), for few trajectories that chain
+// alone.  Measured against the LDS kernel: 128 species x 512
 // reactions, 131072 trajectories of 13350 events 639 -> 168 ms, 64
 // trajectories 217 -> 12 ms; 256 networks x 256 trajectories in one launch
-// 39.1 -> 7.1 ms; 48 x 96 with 53 rate expressions, 32768 trajectories
-// 510 -> 26.8 ms.
+// 39.1 -> 7.3 ms; 48 x 96 with 53 rate expressions, 32768 trajectories
+// 510 -> 26.9 ms.
 #include <hip/hip_runtime.h>
 
 #include "rebop_expr.h"

@@ -255,10 +255,11 @@ __device__ __forceinline__ bool usual_total(double tot) {
   return usual_distance(tot) < kUsualSpan;
 }
 
-// E / tot, correctly rounded, for a usual total: the reciprocal refined by two
-// Newton steps and the quotient corrected by its exact remainder.  These are
-// the operations of the compiler's own division without its scaling and its
-// special cases, which change nothing in this range.
+// E / tot, correctly rounded, for a usual total: Markstein's division, the
+// reciprocal refined by two Newton-Raphson steps and the quotient corrected by
+// its exact remainder (IBM Journal of Research and Development 34, 1990).  The
+// scaling and the special cases of a general division change nothing in this
+// range.
 __device__ __forceinline__ double usual_quotient(double e, double tot) {
   double y = __builtin_amdgcn_rcp(tot);
   y = __builtin_fma(y, __builtin_fma(-tot, y, 1.0), y);

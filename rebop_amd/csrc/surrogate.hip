@@ -335,7 +335,9 @@ __global__ void __launch_bounds__(256) gemm_nt_kernel(int M, int N, int K, const
 // time would leave the chip a quarter full; all of them give 216 tiles (five
 // layers, width 512).  Splits write their sums to part[z], which
 // grad_reduce_kernel adds in order: no atomics, and the same bits every run.
-// Bound by LDS issue.  Five layers of width 512, batch 4096: 23.7 us (a launch
+// Bound by the latency of its loads and LDS accesses (the waves wait 45 % of
+// their time; LDS instructions and their extra cycles take 15 % of the CU
+// cycles).  Five layers of width 512, batch 4096: 23.7 us (a launch
 // and a clear per layer with scattered LDS stores: 113 us; rows padded by four
 // elements instead of the chunk permutation: 29.5 us).
 constexpr int WG_MAXL = 8;
@@ -1179,13 +1181,14 @@ struct NllComp {
 // grad = d(mean NLL over items and samples)/d head (FP32, [B][ldh]);
 // loss_sum += total NLL (FP64).
 //
-// Bound by FP64 issue.  What does not depend on the sample is computed once
+// Bound by FP64 instructions and the latency of their chains (VALU issue on
+// 0.65 of the CU cycles, 54 % of it FP64 arithmetic).  What does not depend on the sample is computed once
 // per (species, component), one lane each, and read back from LDS; per sample
 // and negative binomial the ln Gamma and digamma share their logarithm,
 // reciprocal and shift; the responsibilities come from the exponentials of
 // the log-sum-exp; and the 64-lane sums of the 20 (unbounded: 24) gradient
 // terms halve the number of values per step instead of reducing each alone.
-// Four waves per SIMD (128 VGPRs, 28 bytes of spill) measured 61 us at 4096
+// Four waves per SIMD (128 VGPRs, 28 bytes of spill) measured 62 us at 4096
 // items x 4 species x 64 samples, three 64 us, five 62 us (92 us unbounded),
 // the components unrolled at two 75 us; one wave per item with every term on
 // every lane 235 us, and at 64 items 9 us against 69 us.
