@@ -688,6 +688,7 @@ def main() -> int:
             print(f"step {k}: {st.events} events, {st.kernel_ms:.0f} ms", file=sys.stderr, flush=True)
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
+    kernel_name = _native.last_kernel()
 
     value = events / wall
     out_bytes = wl.output_bytes()
@@ -718,6 +719,7 @@ def main() -> int:
             "trajectories_per_s": trajs / wall,
             "output_gb_per_s": out_bytes * args.steps / wall / 1e9,
             "kernel": sorted(kinds),
+            "kernel_name": kernel_name,
             "autotuned": tuned,
             "device": dev_name,
             "compute_units": cus,
